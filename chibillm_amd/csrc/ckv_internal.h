@@ -126,10 +126,11 @@ constexpr uint32_t max_rope_pairs = 512;
 struct rope_table {
     float inv_freq[max_rope_pairs];
 };
-// The first 64 of them, all that a 128-wide head uses: the fused decode's
+// The first N of them, all that a head of 2N features uses: the fused decode's
 // kernel argument.
-struct rope_table64 {
-    float inv_freq[64];
+template <int N>
+struct rope_pairs {
+    float inv_freq[N];
 };
 
 // One rotary pair (a, b) -> (a cos - b sin, b cos + a sin), written once with

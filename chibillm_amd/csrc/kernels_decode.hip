@@ -1,15 +1,19 @@
 // Paged GQA decode attention.
 //
-// Fast path (head_dim 128, 16-token pages, 1/2/4/8 q heads per KV head; f32
-// pages up to 4): one workgroup per (plan workgroup, kv_head) serves every q
-// head of the KV head's GQA group, so each K/V byte is read once. A wave reads
-// four token rows per load instruction, 16 lanes per row, so lane l holds 8
+// Fast path (head_dim 128 or 256, 16-token pages, 1/2/4/8 q heads per KV head;
+// f32 pages up to 4): one workgroup per (plan workgroup, kv_head) serves every
+// q head of the KV head's GQA group, so each K/V byte is read once. Of 128-wide
+// heads a wave reads four token rows per load instruction, 16 lanes per row, so lane l holds 8
 // features of token 4j + l/16: 8*(l%16).. of a bf16/fp16 row (16 bytes), or
 // 4*(l%16).. and 64 + 4*(l%16).. of an f32 row (two 16-byte words, each
 // instruction reading 256 contiguous bytes). A score is a dot chain over the lane's 8 features
 // (v_dot2 for 16-bit pairs) followed by a 16-lane DPP all-reduce (4 VALU ops).
 // Each 16-lane row group keeps its own online-softmax state over its tokens;
-// the four states are merged once per segment. Scores are kept in the log2
+// the four states are merged once per segment. 256-wide heads take 32 lanes a
+// row, two rows per load instruction and half a page per step, which keeps the
+// registers of the 128-wide form; they are read once for the whole group
+// instead of once per q head by one wave (the general path): 32 rows of
+// U[256, 4096] tokens, 2 kv heads, 8 q heads, rotated and gated, 607 -> 57 us. Scores are kept in the log2
 // domain (scale * log2(e)) so every exponential is one v_exp_f32. Rows the
 // batch plan cuts are merged in the same launch with weights 2^(m_c - M), the
 // reduction of paged_attention_reduce_f32
@@ -42,51 +46,52 @@ __device__ __forceinline__ uint4 load_stream(const void* p)
     return make_uint4(t.x, t.y, t.z, t.w);
 }
 
-// The eight elements of one K, V or query head row a lane of the fast decode
-// holds: lane part p (of 16) takes the 16 bytes at 16p, features 8p..8p+7 of
-// a 16-bit row; of an f32 row (the reference's storage,
-// src/metal/metal_kv_cache.cc:57-69) also the 16 bytes at 256 + 16p, so its
-// features are 4p..4p+3 and 64+4p..64+4p+3. Either way each 16-byte load
-// instruction of 16 lanes reads 256 contiguous bytes of the row.
-template <int DT>
+// The eight elements of one K, V or query head row (D features) a lane of the
+// fast decode holds: lane part p (of D / 8) takes the 16 bytes at 16p, features
+// 8p..8p+7 of a 16-bit row; of an f32 row (the reference's storage,
+// src/metal/metal_kv_cache.cc:57-69) also the 16 bytes at 2D + 16p, so its
+// features are 4p..4p+3 and D/2+4p..D/2+4p+3. Either way each 16-byte load
+// instruction of D / 8 lanes reads 2D contiguous bytes of the row.
+template <int DT, int D>
 struct lane8 {
+    static constexpr int dtype = DT;
     static constexpr uint32_t words = DT == CKV_F32 ? 2 : 1;
     static constexpr uint32_t elem = DT == CKV_F32 ? 4 : 2; // bytes per element
-    static constexpr uint32_t stride = 256;                 // bytes between the words
+    static constexpr uint32_t stride = 2 * D;               // bytes between the words
     uint4 w[words];
     // the head feature of the lane's element i (of 8), for lane part p
     static __device__ __forceinline__ uint32_t feature(uint32_t p, uint32_t i)
     {
-        return DT == CKV_F32 ? (i < 4 ? 4 * p + i : 64 + 4 * p + (i - 4)) : 8 * p + i;
+        return DT == CKV_F32 ? (i < 4 ? 4 * p + i : D / 2 + 4 * p + (i - 4)) : 8 * p + i;
     }
 };
 
-template <int DT>
-__device__ __forceinline__ lane8<DT> load8_stream(const char* p)
+template <class Row>
+__device__ __forceinline__ Row load8_stream(const char* p)
 {
-    lane8<DT> x;
+    Row x;
 #pragma unroll
-    for (uint32_t i = 0; i < lane8<DT>::words; ++i)
-        x.w[i] = load_stream(p + lane8<DT>::stride * i);
+    for (uint32_t i = 0; i < Row::words; ++i)
+        x.w[i] = load_stream(p + Row::stride * i);
     return x;
 }
 
-template <int DT>
-__device__ __forceinline__ lane8<DT> load8(const char* p)
+template <class Row>
+__device__ __forceinline__ Row load8(const char* p)
 {
-    lane8<DT> x;
+    Row x;
 #pragma unroll
-    for (uint32_t i = 0; i < lane8<DT>::words; ++i)
-        x.w[i] = *reinterpret_cast<const uint4*>(p + lane8<DT>::stride * i);
+    for (uint32_t i = 0; i < Row::words; ++i)
+        x.w[i] = *reinterpret_cast<const uint4*>(p + Row::stride * i);
     return x;
 }
 
-template <int DT>
-__device__ __forceinline__ void store8(char* p, const lane8<DT>& x)
+template <class Row>
+__device__ __forceinline__ void store8(char* p, const Row& x)
 {
 #pragma unroll
-    for (uint32_t i = 0; i < lane8<DT>::words; ++i)
-        *reinterpret_cast<uint4*>(p + lane8<DT>::stride * i) = x.w[i];
+    for (uint32_t i = 0; i < Row::words; ++i)
+        *reinterpret_cast<uint4*>(p + Row::stride * i) = x.w[i];
 }
 
 __device__ __forceinline__ float fast_exp2(float x)
@@ -227,6 +232,22 @@ __device__ __forceinline__ float row16_sum(float v)
     return v;
 }
 
+// Sum over each group of LANES lanes (16 or 32), result in every lane of it.
+// v_permlane16_swap of a value with itself leaves the even 16-lane row of each
+// pair in one result and the odd row in the other, in both rows.
+template <uint32_t LANES>
+__device__ __forceinline__ float lanes_sum(float v)
+{
+    static_assert(LANES == 16 || LANES == 32);
+    v = row16_sum(v);
+    if constexpr (LANES == 32) {
+        const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+        const auto sw = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+        v = __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
+    }
+    return v;
+}
+
 // Partial record per (work item, q head): [max, denominator, 0, 0, acc[D]].
 __host__ __device__ constexpr uint32_t record_floats(uint32_t head_dim)
 {
@@ -250,9 +271,10 @@ __host__ __device__ constexpr bool fast_fits(uint32_t group, int dtype)
 
 // q . k over a lane's eight elements (16-bit pairs by v_dot2 with fp32
 // accumulation; f32 by fused multiply-adds), and a V row widened to floats.
-template <int DT>
-__device__ __forceinline__ float dot8(const lane8<DT>& q, const lane8<DT>& k)
+template <class Row>
+__device__ __forceinline__ float dot8(const Row& q, const Row& k)
 {
+    constexpr int DT = Row::dtype;
     if constexpr (DT == CKV_F32) {
         float d = 0.0f;
 #pragma unroll
@@ -272,9 +294,10 @@ __device__ __forceinline__ float dot8(const lane8<DT>& q, const lane8<DT>& k)
     }
 }
 
-template <int DT>
-__device__ __forceinline__ void widen8(const lane8<DT>& v, float (&f)[8])
+template <class Row>
+__device__ __forceinline__ void widen8(const Row& v, float (&f)[8])
 {
+    constexpr int DT = Row::dtype;
     if constexpr (DT == CKV_F32) {
 #pragma unroll
         for (uint32_t i = 0; i < 2; ++i) {
@@ -327,7 +350,8 @@ __device__ __forceinline__ void store_elem(void* base, uint64_t i, float x)
 // scalar table read per page); the next page's K/V loads are issued before the
 // current page is processed. Lane 16*group + part reads features 8*part..8*part+7 of token
 // 4j + group of the page (j = 0..3): four 1 KiB wave loads per page for K and
-// four for V. The wave's four row-group softmax states are merged with
+// four for V (256-wide heads: lane 32*group + part, token 2j + group of half a
+// page; pages below stand for these units). The wave's four row-group softmax states are merged with
 // shuffles, the W wave states through LDS, and the workgroup writes the
 // normalised output of the group's q heads. GATED multiplies it by
 // sigmoid(gate) first; the gate values are loaded when the workgroup starts,
@@ -341,21 +365,25 @@ __device__ __forceinline__ void store_elem(void* base, uint64_t i, float x)
 // queries and the new token's key by the row's position first, as rope_f32
 // (src/metal/kernels/tensor_ops.metal:158-195) would: feature f < rotary/2
 // pairs with f + rotary/2, which sits in the lane part ^ (rotary/16) of the
-// same 16-lane group, so one lane exchange per register rotates a head.
-template <int G, int DT, bool FUSED, bool GATED, bool ROPE>
+// same row's lanes, so one lane exchange per register rotates a head.
+template <int D, int G, int DT, bool FUSED, bool GATED, bool ROPE>
 __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ? 2 : 4) void decode_wg_kernel(
     pool_view p, meta_view m, uint32_t layer, const char* __restrict__ q, uint32_t q_heads,
     float scale_log2, void* __restrict__ out, const char* __restrict__ k_in,
-    const char* __restrict__ v_in, const void* __restrict__ gate, rope_table64 freq,
+    const char* __restrict__ v_in, const void* __restrict__ gate, rope_pairs<D / 2> freq,
     uint32_t rotary, split_scratch split, uint32_t group_stride, uint32_t head_base)
 {
     static_assert(!(ROPE && DT == CKV_F32), "the fused rotation works on 16-bit pairs");
     constexpr bool F16 = DT == CKV_F16;
     using ops = half2_ops<F16>;
-    using row8 = lane8<DT>;
+    using row8 = lane8<DT, D>;
     constexpr uint32_t ES = row8::elem;
-    constexpr uint32_t D = 128;
     constexpr uint32_t BS = 16;
+    // A wave reads ROWS token rows of LANES lanes per load instruction, and a
+    // unit of UT tokens (a page, or half of one of 256-wide heads) with four.
+    constexpr uint32_t LANES = D / 8, ROWS = 64 / LANES;
+    constexpr uint32_t UT = 4 * ROWS, UPP = BS / UT; // units per page
+    static_assert(UT * UPP == BS);
     extern __shared__ float lds[];
     const uint32_t W = blockDim.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // a scalar
@@ -381,16 +409,16 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         uint32_t lane;
         asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
         const uint32_t tid = wave * 64 + lane;
-        const uint32_t group = lane >> 4;
-        const uint32_t part = lane & 15;
+        const uint32_t group = lane / LANES;
+        const uint32_t part = lane % LANES;
         const uint32_t head_off = kv_head * (D * ES) + part * 16u; // the lane's first word
         const uint32_t row = e0.x;
         const uint32_t chunk = e0.y;
         const uint32_t position = e0.z;
-        const uint32_t n_pages = position / BS + 1;
-        const uint32_t last_in_page = position % BS;
+        const uint32_t u_last = position / UT; // the row's last unit
+        const uint32_t last_in_unit = position % UT;
         const uint32_t pg_first = e1.x;
-        const uint32_t pg_end = e1.y;
+        const uint32_t u_end = UPP == 1 ? e1.y : min(e1.y * UPP, u_last + 1);
         const uint32_t n_chunks = e1.z;
         float gate_early = 0.0f; // the first epilogue iteration's gate value (one register)
         if constexpr (GATED) {
@@ -402,26 +430,30 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         row8 qv[G];
 #pragma unroll
         for (int g = 0; g < G; ++g)
-            qv[g] = load8<DT>(q + ((uint64_t)row * q_heads + qh0 + g) * D * ES + part * 16);
+            qv[g] = load8<row8>(q + ((uint64_t)row * q_heads + qh0 + g) * D * ES + part * 16);
 
         // ROPE: this lane's 8 features (pairs j0 .. j0 + 7) and their rotation;
         // every lane of the wave takes part in the exchanges. The queries and the
         // new token's key share the row's position: both are rotated while the
         // wave's first page loads, and the rotated key (this lane's 16 bytes of
         // it) takes the new token's place when the last page is processed. The
-        // row's rotary/2 angles are computed once, by wave 0, into LDS past the
-        // merge area.
+        // row's rotary/2 angles are computed once, by wave 0 (and 1), into LDS past
+        // the merge area.
         const uint32_t rot_mask = ROPE ? rotary / 16 : 1; // lane parts per half of the rotary width
         const bool rot_on = ROPE && part < 2 * rot_mask;
         const bool rot_first = part < rot_mask;
         auto angles = [&](float (&rc)[8], float (&rs)[8]) {
             float* table = lds + W * G * (D + 2); // (cos, sin) per pair
-            if (wave == 0 && lane < rotary / 2) {
+            auto angle = [&](uint32_t j) {
                 float sn, cs;
-                sincosf(static_cast<float>(position) * freq.inv_freq[lane], &sn, &cs);
-                table[2 * lane] = cs;
-                table[2 * lane + 1] = sn;
-            }
+                sincosf(static_cast<float>(position) * freq.inv_freq[j], &sn, &cs);
+                table[2 * j] = cs;
+                table[2 * j + 1] = sn;
+            };
+            if (wave == 0 && lane < rotary / 2)
+                angle(lane);
+            if (D > 128 && wave == (W > 1) && 64 + lane < rotary / 2)
+                angle(64 + lane);
             __syncthreads();
             const uint32_t j0 = 8 * (part & (rot_mask - 1));
 #pragma unroll
@@ -453,7 +485,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         const uint64_t in_row = (uint64_t)row * row_bytes + head_off;
         uint4 k_new = make_uint4(0, 0, 0, 0); // ROPE: the new token's key, rotated once loaded
         if constexpr (ROPE)
-            k_new = load8<DT>(k_in + in_row).w[0];
+            k_new = load8<row8>(k_in + in_row).w[0];
 
         float mx[G], den[G], acc[G][8];
 #pragma unroll
@@ -466,54 +498,55 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         }
 
         // rows past the row's last token re-read that token (in bounds, written)
-        auto load_page = [&](uint32_t pg, row8* k, row8* v) {
-            const uint64_t base = (uint64_t)tbl[pg] * page_bytes;
+        auto load_unit = [&](uint32_t u, row8* k, row8* v) {
+            const uint64_t base = (uint64_t)tbl[u / UPP] * page_bytes;
+            const uint32_t t0 = u % UPP * UT; // the unit's first token in its page
             const char* kb = kl + base;
             const char* vb = vl + base;
-            const bool last_page = pg == n_pages - 1;
-            const uint32_t last = last_page ? last_in_page : BS - 1;
+            const bool last_unit = u == u_last;
+            const uint32_t last = last_unit ? last_in_unit : UT - 1;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const uint32_t r = min(4u * j + group, last);
-                const uint32_t off = r * row_bytes + head_off;
-                const bool fresh = FUSED && last_page && r == last_in_page;
+                const uint32_t r = min(ROWS * j + group, last);
+                const uint32_t off = (t0 + r) * row_bytes + head_off;
+                const bool fresh = FUSED && last_unit && r == last_in_unit;
                 // ROPE: the new token's slot is read too and replaced in process
-                k[j] = load8_stream<DT>(fresh && !ROPE ? k_in + in_row : kb + off);
-                v[j] = load8_stream<DT>(fresh ? v_in + in_row : vb + off);
+                k[j] = load8_stream<row8>(fresh && !ROPE ? k_in + in_row : kb + off);
+                v[j] = load8_stream<row8>(fresh ? v_in + in_row : vb + off);
             }
         };
 
-        auto process = [&](row8* k, const row8* v, uint32_t pg) {
-            const uint32_t valid = pg == n_pages - 1 ? last_in_page + 1 : BS;
-            if (FUSED && pg == n_pages - 1) {
+        auto process = [&](row8* k, const row8* v, uint32_t u) {
+            const uint32_t valid = u == u_last ? last_in_unit + 1 : UT;
+            if (FUSED && u == u_last) {
                 if constexpr (ROPE) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        if (4u * j + group == last_in_page)
+                        if (ROWS * j + group == last_in_unit)
                             k[j].w[0] = k_new;
                 }
                 // append: the lanes holding the new token write it into its slot
-                const uint64_t base = (uint64_t)tbl[pg] * page_bytes;
-                const uint32_t off = last_in_page * row_bytes + head_off;
+                const uint64_t base = (uint64_t)tbl[u / UPP] * page_bytes;
+                const uint32_t off = (u % UPP * UT + last_in_unit) * row_bytes + head_off;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    if (4u * j + group == last_in_page) {
-                        store8<DT>(const_cast<char*>(kl) + base + off, k[j]);
-                        store8<DT>(const_cast<char*>(vl) + base + off, v[j]);
+                    if (ROWS * j + group == last_in_unit) {
+                        store8(const_cast<char*>(kl) + base + off, k[j]);
+                        store8(const_cast<char*>(vl) + base + off, v[j]);
                     }
                 }
             }
             bool ok[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                ok[j] = 4u * j + group < valid;
+                ok[j] = ROWS * j + group < valid;
             float pw[G][4];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 float s[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float r = row16_sum(dot8<DT>(qv[g], k[j])) * scale_log2;
+                    const float r = lanes_sum<LANES>(dot8(qv[g], k[j])) * scale_log2;
                     s[j] = ok[j] ? r : -INFINITY;
                 }
                 const float nm = fmaxf(mx[g], fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
@@ -535,7 +568,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float vf[8];
-                widen8<DT>(v[j], vf);
+                widen8(v[j], vf);
 #pragma unroll
                 for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -545,9 +578,9 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         };
 
         row8 ka[4], va[4], kb[4], vb[4];
-        uint32_t pg = pg_first + wave;
-        if (pg < pg_end)
-            load_page(pg, ka, va);
+        uint32_t u = pg_first * UPP + wave;
+        if (u < u_end)
+            load_unit(u, ka, va);
         // ROPE: rotate the queries and the new key while the first page loads
         if constexpr (ROPE) {
             float rc[8], rs[8];
@@ -581,38 +614,42 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                 break;
             }
         };
-        while (pg < pg_end) {
-            uint32_t next = pg + W;
+        while (u < u_end) {
+            uint32_t next = u + W;
             rotate_priority();
-            if (next < pg_end)
-                load_page(next, kb, vb);
-            process(ka, va, pg);
-            pg = next;
-            if (pg >= pg_end)
+            if (next < u_end)
+                load_unit(next, kb, vb);
+            process(ka, va, u);
+            u = next;
+            if (u >= u_end)
                 break;
-            next = pg + W;
+            next = u + W;
             rotate_priority();
-            if (next < pg_end)
-                load_page(next, ka, va);
-            process(kb, vb, pg);
-            pg = next;
+            if (next < u_end)
+                load_unit(next, ka, va);
+            process(kb, vb, u);
+            u = next;
         }
         __builtin_amdgcn_s_setprio(0); // the merge at the default priority
 
-        // merge the wave's four row-group states (lanes l, l^16, l^32, l^48)
+        // merge the wave's row-group states (lanes l, l ^ LANES, ... l ^ 32)
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            float M = fmaxf(mx[g], __shfl_xor(mx[g], 16));
-            M = fmaxf(M, __shfl_xor(M, 32));
+            float M = mx[g];
+#pragma unroll
+            for (uint32_t x = LANES; x < 64; x *= 2)
+                M = fmaxf(M, __shfl_xor(M, x));
             const float w = mx[g] == -INFINITY ? 0.0f : fast_exp2(mx[g] - M);
             float d = den[g] * w;
-            d += __shfl_xor(d, 16);
-            d += __shfl_xor(d, 32);
+#pragma unroll
+            for (uint32_t x = LANES; x < 64; x *= 2)
+                d += __shfl_xor(d, x);
 #pragma unroll
             for (int f = 0; f < 8; ++f) {
                 float a = acc[g][f] * w;
-                a += __shfl_xor(a, 16);
-                a += __shfl_xor(a, 32);
+#pragma unroll
+                for (uint32_t x = LANES; x < 64; x *= 2)
+                    a += __shfl_xor(a, x);
                 acc[g][f] = a;
             }
             den[g] = d;
@@ -1006,7 +1043,7 @@ uint32_t fast_waves(uint32_t group, int dtype, uint32_t units, int cu_count,
     return limit;
 }
 
-template <int G>
+template <int D, int G>
 hipError_t launch_fast(hipStream_t s, const pool_view& p, const meta_view& m, uint32_t layer,
                        const void* q, uint32_t q_heads, float scale_log2, void* out, int dt,
                        const void* k_in, const void* v_in, const void* gate, int cu_count,
@@ -1020,10 +1057,10 @@ hipError_t launch_fast(hipStream_t s, const pool_view& p, const meta_view& m, ui
         // pass holds twice the registers its 512-lane workgroups allow); each
         // reads the K/V once more, the fused append writes the same token twice
         if (dt == CKV_F32) {
-            hipError_t e = launch_fast<4>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in,
+            hipError_t e = launch_fast<D, 4>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in,
                                           v_in, gate, cu_count, split, rope, rotary, 8, 0);
             if (e == hipSuccess)
-                e = launch_fast<4>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in, v_in,
+                e = launch_fast<D, 4>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in, v_in,
                                    gate, cu_count, split, rope, rotary, 8, 4);
             return e;
         }
@@ -1032,14 +1069,14 @@ hipError_t launch_fast(hipStream_t s, const pool_view& p, const meta_view& m, ui
     const uint32_t waves = fast_waves(G, dt, units, cu_count, m.mean_pages, m.split_pages);
     const dim3 grid(units), block(64 * waves);
     // the merge's (acc, max, denominator) per wave, then the rope angle table
-    const size_t lds = ((size_t)waves * G * (128 + 2) + (rope ? 2 * 64 : 0)) * sizeof(float);
+    const size_t lds = ((size_t)waves * G * (D + 2) + (rope ? rotary : 0)) * sizeof(float);
     const auto qq = static_cast<const char*>(q);
     const auto ki = static_cast<const char*>(k_in);
     const auto vi = static_cast<const char*>(v_in);
-    rope_table64 f64 = {};
+    rope_pairs<D / 2> freq = {};
     if (rope)
         for (uint32_t j = 0; j < rotary / 2; ++j)
-            f64.inv_freq[j] = rope->inv_freq[j];
+            freq.inv_freq[j] = rope->inv_freq[j];
     // one instantiation per (dtype, fused, gated, rope); rope only when fused
     // and on 16-bit pages
     const int variant = (rope ? 16 : 0) | (dt << 2) | (k_in ? 2 : 0) | (gate ? 1 : 0);
@@ -1047,8 +1084,8 @@ hipError_t launch_fast(hipStream_t s, const pool_view& p, const meta_view& m, ui
 #define CKV_FAST_CASE(DT_, FUSED_, GATED_, ROPE_)                                              \
     case (ROPE_ ? 16 : 0) | (DT_ << 2) | (FUSED_ ? 2 : 0) | (GATED_ ? 1 : 0):                  \
         if constexpr (fast_fits(G, DT_))                                                       \
-            decode_wg_kernel<G, DT_, FUSED_, GATED_, ROPE_><<<grid, block, lds, s>>>(          \
-                p, m, layer, qq, q_heads, scale_log2, out, ki, vi, gate, f64, rotary, split,   \
+            decode_wg_kernel<D, G, DT_, FUSED_, GATED_, ROPE_><<<grid, block, lds, s>>>(       \
+                p, m, layer, qq, q_heads, scale_log2, out, ki, vi, gate, freq, rotary, split,  \
                 group_stride, head_base);                                                      \
         else                                                                                   \
             return hipErrorInvalidValue;                                                       \
@@ -1074,6 +1111,28 @@ hipError_t launch_fast(hipStream_t s, const pool_view& p, const meta_view& m, ui
         return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+// The instantiation for a head width and a GQA group that decode_uses_fast_path admits.
+template <int D, class... Args>
+hipError_t launch_group(uint32_t group, const Args&... args)
+{
+    switch (group) {
+    case 1:
+        return launch_fast<D, 1>(args...);
+    case 2:
+        return launch_fast<D, 2>(args...);
+    case 4:
+        return launch_fast<D, 4>(args...);
+    default:
+        return launch_fast<D, 8>(args...);
+    }
+}
+
+template <class... Args>
+hipError_t launch_width(uint32_t head_dim, uint32_t group, const Args&... args)
+{
+    return head_dim == 256 ? launch_group<256>(group, args...) : launch_group<128>(group, args...);
 }
 
 // Pages of a row at `position`, and the batch's total and longest.
@@ -1393,7 +1452,7 @@ bool decode_uses_fast_path(const pool_view& p, uint32_t q_heads)
 {
     const uint32_t G = q_heads / p.kv_heads;
     // f32 at G = 8 runs as two passes of G = 4 (launch_fast<8>)
-    return p.head_dim == 128 && p.block_size == 16
+    return (p.head_dim == 128 || p.head_dim == 256) && p.block_size == 16
         && (G == 1 || G == 2 || G == 4 || G == 8)
         && (fast_fits(G, p.dtype) || (G == 8 && p.dtype == CKV_F32)) && aligned16(p.keys)
         && aligned16(p.values);
@@ -1412,21 +1471,9 @@ hipError_t launch_decode(hipStream_t s, const pool_view& p, const meta_view& m, 
         return hipSuccess;
     const float scale_log2 = scale * log2e;
     if (decode_fast_applies(p, q_heads, q, out)) {
-        const int dt = p.dtype;
-        switch (q_heads / p.kv_heads) {
-        case 1:
-            return launch_fast<1>(s, p, m, layer, q, q_heads, scale_log2, out, dt, nullptr,
-                                  nullptr, gate, cu_count, split);
-        case 2:
-            return launch_fast<2>(s, p, m, layer, q, q_heads, scale_log2, out, dt, nullptr,
-                                  nullptr, gate, cu_count, split);
-        case 4:
-            return launch_fast<4>(s, p, m, layer, q, q_heads, scale_log2, out, dt, nullptr,
-                                  nullptr, gate, cu_count, split);
-        default:
-            return launch_fast<8>(s, p, m, layer, q, q_heads, scale_log2, out, dt, nullptr,
-                                  nullptr, gate, cu_count, split);
-        }
+        const void* no_row = nullptr;
+        return launch_width(p.head_dim, q_heads / p.kv_heads, s, p, m, layer, q, q_heads,
+                            scale_log2, out, p.dtype, no_row, no_row, gate, cu_count, split);
     }
     if (p.head_dim > 64u * generic_max_features_per_lane)
         return hipErrorInvalidValue;
@@ -1456,24 +1503,11 @@ hipError_t launch_append_decode(hipStream_t s, const pool_view& p, const meta_vi
 {
     if (!m.rows)
         return hipSuccess;
-    if (rope && (rotary < 16 || rotary > 128 || (rotary & (rotary - 1)) != 0))
+    if (rope && (rotary < 16 || rotary > p.head_dim || (rotary & (rotary - 1)) != 0))
         return hipErrorInvalidValue;
     const float scale_log2 = scale * log2e;
-    const int dt = p.dtype;
-    switch (q_heads / p.kv_heads) {
-    case 1:
-        return launch_fast<1>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in, v_in, gate,
-                              cu_count, split, rope, rotary);
-    case 2:
-        return launch_fast<2>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in, v_in, gate,
-                              cu_count, split, rope, rotary);
-    case 4:
-        return launch_fast<4>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in, v_in, gate,
-                              cu_count, split, rope, rotary);
-    default:
-        return launch_fast<8>(s, p, m, layer, q, q_heads, scale_log2, out, dt, k_in, v_in, gate,
-                              cu_count, split, rope, rotary);
-    }
+    return launch_width(p.head_dim, q_heads / p.kv_heads, s, p, m, layer, q, q_heads, scale_log2,
+                        out, p.dtype, k_in, v_in, gate, cu_count, split, rope, rotary);
 }
 
 hipError_t launch_merge(hipStream_t s, const pool_view& p, const meta_view& m, uint32_t q_heads,

@@ -277,7 +277,7 @@ int ckv_gather(ckv_pool* pool, size_t layer, size_t table_offset, size_t table_l
  * out = softmax(q . k * scale) . v with fp32 accumulation. queries and
  * output are device [rows, q_heads*head_dim] of the pool dtype.
  * Decode form: the q heads of a GQA group share every K/V read. Pools with
- * head_dim 128, 16-token pages and 1, 2, 4 or 8 q heads per kv head (f32 pools
+ * head_dim 128 or 256, 16-token pages and 1, 2, 4 or 8 q heads per kv head (f32 pools
  * with 8 in two passes of 4) take one workgroup per (row, kv_head),
  * or per page chunk of rows the batch plan cuts (ckv_decode_plan), the chunks
  * merged by the last to finish; other geometries take split-KV over token
@@ -391,7 +391,7 @@ int ckv_rope_append(ckv_pool* pool, size_t layer, const void* keys, const void* 
  * sigmoid_mul) — src/qwen/qwen_layer.cc:20-30, :43-49 (Qwen3) and :183-206
  * (Qwen3.5 full attention) — in one launch where ckv_append_decode's fused
  * kernel applies, the pool is bf16 or fp16 and rotary_dim (0 = head_dim) is
- * 16, 32, 64 or 128; otherwise
+ * 16, 32, 64, 128 or 256; otherwise
  * as ckv_rope into a pool-owned buffer, ckv_rope_append and the attention.
  * keys/values: [rows, kv_heads*head_dim]; queries: [rows, q_heads*head_dim];
  * queries and keys are read unrotated and not modified; gate may be NULL (no

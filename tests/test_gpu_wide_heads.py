@@ -1,0 +1,125 @@
+"""Attention over 256-wide heads against the oracle (rope_f32, store_kv, paged
+attention, gate) and against the general path, which misaligned queries take.
+
+Pages hold NaN wherever no token was written, so a read past a row's tokens
+shows in the output. Rows end at and around the edges of a page and of the
+half page a wave reads at a time."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from tests.gpu_util import (approx, assert_close, force_plan, new_context, new_pool, to_dev,
+                            to_host)
+
+pytestmark = pytest.mark.gpu
+
+D = 256
+LENGTHS = [1, 2, 7, 8, 9, 15, 16, 17, 24, 25, 160, 161, 401, 700]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = new_context()
+    yield c
+    c.sync()
+    c.close()
+
+
+def nan_pages(code, n):
+    if code == orc.F32:
+        return np.full(n, np.nan, np.float32)
+    return np.full(n, 0x7FC0 if code == orc.BF16 else 0x7E00, np.uint16)
+
+
+def misaligned(t):
+    """A copy one element past a 16-byte boundary."""
+    base = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    view = base[1:1 + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("code,group,rotary,gated,split", [
+    (orc.BF16, 4, 64, True, None), (orc.BF16, 4, 256, False, "0"), (orc.F16, 4, 128, True, "3"),
+    (orc.BF16, 2, 64, True, "b6"), (orc.F16, 1, 16, False, "1"), (orc.BF16, 8, 256, True, "5"),
+    (orc.BF16, 2, None, False, "2"), (orc.F32, 4, None, True, "4"), (orc.F32, 8, None, False, "2"),
+    (orc.F32, 1, 64, False, None), (orc.BF16, 4, 48, False, None)])
+def test_wide_decode_matches_oracle_and_general_path(ctx, code, group, rotary, gated, split,
+                                                     monkeypatch):
+    print(f"wide decode dtype {code} group {group} rotary {rotary} gated {gated} split {split}",
+          flush=True)
+    force_plan(monkeypatch, split)
+    rng = orc.Mt64(900 + 10 * group + code)
+    H = 2
+    Hq, rows, theta = H * group, len(LENGTHS), 1e7
+    pages = [-(-n // 16) for n in LENGTHS]
+    blocks = sum(pages) + 3
+    order = rng.permutation(blocks)
+    tables = np.split(order[:sum(pages)], np.cumsum(pages)[:-1])
+    flat, offsets = np.concatenate(tables), np.cumsum([0] + pages[:-1])
+    positions = [n - 1 for n in LENGTHS]
+    slots = [orc.slot(t, p, 16) for t, p in zip(tables, positions)]
+    geom, F = (1, blocks, 16, H, D), H * D
+    kc, vc = nan_pages(code, blocks * 16 * F), nan_pages(code, blocks * 16 * F)
+    for t, n in zip(tables, LENGTHS):
+        held = [orc.slot(t, p, 16) for p in range(n - 1)]
+        if held:
+            orc.store_kv(kc, vc, rng.normal(len(held) * F, code).reshape(-1, F),
+                         rng.normal(len(held) * F, code).reshape(-1, F), held, 0, blocks * 16)
+    q = rng.normal(rows * Hq * D, code).reshape(rows, Hq * D)
+    kn, vn = (rng.normal(rows * F, code).reshape(rows, F) for _ in range(2))
+    gate = rng.normal(rows * Hq * D, code).reshape(rows, Hq * D) if gated else None
+    scale = float(np.float32(1 / math.sqrt(D)))
+
+    outs, caches = [], []
+    for shift in (lambda t: t, misaligned):
+        pool, kd, vd = new_pool(ctx, geom, code)
+        kd.copy_(to_dev(kc, code))
+        vd.copy_(to_dev(vc, code))
+        pool.upload(flat, offsets, pages, positions, slots)
+        qd, knd, vnd = shift(to_dev(q, code)), to_dev(kn, code), to_dev(vn, code)
+        gd = to_dev(gate, code) if gated else None
+        out = shift(torch.full((rows, Hq * D), float("nan"), dtype=qd.dtype, device="cuda"))
+        if rotary is not None:
+            pool.rope_append_decode(0, knd, vnd, qd, Hq, scale, theta, out, rotary, gd)
+        elif gated:
+            pool.append_decode_gated(0, knd, vnd, qd, Hq, scale, gd, out)
+        else:
+            pool.append_decode(0, knd, vnd, qd, Hq, scale, out)
+        ctx.sync()
+        outs.append(to_host(out, code))
+        caches.append((to_host(kd, code), to_host(vd, code)))
+        if rotary is None and not gated:  # the unfused call over the same pages
+            again = torch.full_like(out, float("nan"))
+            pool.decode(0, qd, Hq, scale, again)
+            ctx.sync()
+            assert np.array_equal(to_host(again, code), outs[-1])
+        pool.close()
+
+    want_k, want_v = kc.copy(), vc.copy()
+    rk = kn if rotary is None else orc.rope(kn, code, H, positions, theta, rotary)
+    orc.store_kv(want_k, want_v, rk, vn, slots, 0, blocks * 16)
+    for got_k, got_v in caches:
+        assert np.array_equal(got_v.view(np.uint8), want_v.view(np.uint8))
+        if rotary is None:
+            assert np.array_equal(got_k.view(np.uint8), want_k.view(np.uint8))
+        elif code == orc.F32:
+            assert np.allclose(got_k, want_k, rtol=1e-5, atol=1e-5, equal_nan=True)
+        else:  # a rotated element within one unit in the last place (sign and magnitude)
+            a, b = (np.where(x & 0x8000, -(x & 0x7FFF).astype(np.int32), x & 0x7FFF)
+                    for x in (got_k.astype(np.int32), want_k.astype(np.int32)))
+            assert np.abs(a - b).max() <= 1
+    rq = q if rotary is None else orc.rope(q, code, Hq, positions, theta, rotary)
+    expected = orc.Attention(geom, caches[0][0], caches[0][1], code, rq, code, positions, flat,
+                             offsets, pages, Hq, 0, scale).online_threads(8)
+    if gated:
+        g = gate if code == orc.F32 else orc.to_f32(gate, code)
+        expected = expected * (1.0 / (1.0 + np.exp(-np.asarray(g, np.float64))))
+    for got, what in zip(outs, ("fast", "general")):
+        if code == orc.F32:
+            assert approx(got, expected, 3e-5, 1.0), what
+        else:
+            assert_close(orc.to_f32(got, code), expected, what=what)
