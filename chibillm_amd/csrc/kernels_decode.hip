@@ -232,20 +232,49 @@ __device__ __forceinline__ float row16_sum(float v)
     return v;
 }
 
+// A value combined with the one 32 (16) lanes away, in every lane.
+template <class Op>
+__device__ __forceinline__ float swap32(float v, Op op)
+{
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto sw = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return op(__builtin_bit_cast(float, (uint32_t)sw[0]), __builtin_bit_cast(float, (uint32_t)sw[1]));
+}
+
+template <class Op>
+__device__ __forceinline__ float swap16(float v, Op op)
+{
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto sw = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return op(__builtin_bit_cast(float, (uint32_t)sw[0]), __builtin_bit_cast(float, (uint32_t)sw[1]));
+}
+
 // Sum over each group of LANES lanes (16 or 32), result in every lane of it.
-// v_permlane16_swap of a value with itself leaves the even 16-lane row of each
-// pair in one result and the odd row in the other, in both rows.
 template <uint32_t LANES>
 __device__ __forceinline__ float lanes_sum(float v)
 {
     static_assert(LANES == 16 || LANES == 32);
     v = row16_sum(v);
-    if constexpr (LANES == 32) {
-        const uint32_t bits = __builtin_bit_cast(uint32_t, v);
-        const auto sw = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
-        v = __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
-    }
+    if constexpr (LANES == 32)
+        v = swap16(v, [](float a, float b) { return a + b; });
     return v;
+}
+
+// Of two values the sums over lanes l and l ^ 32: a's in lanes 0..31, b's in
+// lanes 32..63 (the swap exchanges a's upper half with b's lower one); and
+// over lanes l and l ^ 16: a's in the even rows of 16 lanes, b's in the odd.
+__device__ __forceinline__ float scatter32(float a, float b)
+{
+    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a),
+                                                     __builtin_bit_cast(uint32_t, b), false, false);
+    return __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
+}
+
+__device__ __forceinline__ float scatter16(float a, float b)
+{
+    const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a),
+                                                     __builtin_bit_cast(uint32_t, b), false, false);
+    return __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
 }
 
 // Partial record per (work item, q head): [max, denominator, 0, 0, acc[D]].
@@ -632,25 +661,35 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         }
         __builtin_amdgcn_s_setprio(0); // the merge at the default priority
 
-        // merge the wave's row-group states (lanes l, l ^ LANES, ... l ^ 32)
+        // What follows bounds small batches: a launch over six rows of up to
+        // 1,500 tokens has its last page scored after 5.5 us and ended at
+        // 10.9, waiting on one LDS or memory round trip after another. With
+        // the swaps below and the reads of the merges four at a time a layer
+        // of that batch takes 11.5 us instead of 12.9, four rows of U[64, 512]
+        // 9.3 instead of 10.4, one 32K row 30.3 instead of 31.4 (launch gaps
+        // included, rotated).
+        // Merge the wave's row-group states. The maxima and denominators are
+        // reduced into every lane; the accumulators are reduced and scattered,
+        // each swap halving what a lane holds: of its features 0..7 a lane of
+        // half h keeps 4h..4h+3 after the 32-lane swap, and with four groups
+        // the two at 2 * (group % 2) of those after the 16-lane one.
+        constexpr uint32_t KEEP = ROWS == 4 ? 2 : 4;
+        const uint32_t kept = 4 * (lane >> 5) + (ROWS == 4 ? 2 * (group & 1) : 0);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            float M = mx[g];
-#pragma unroll
-            for (uint32_t x = LANES; x < 64; x *= 2)
-                M = fmaxf(M, __shfl_xor(M, x));
+            float M = swap32(mx[g], [](float a, float b) { return fmaxf(a, b); });
+            if constexpr (ROWS == 4)
+                M = swap16(M, [](float a, float b) { return fmaxf(a, b); });
             const float w = mx[g] == -INFINITY ? 0.0f : fast_exp2(mx[g] - M);
-            float d = den[g] * w;
+            float d = swap32(den[g] * w, [](float a, float b) { return a + b; });
+            if constexpr (ROWS == 4)
+                d = swap16(d, [](float a, float b) { return a + b; });
 #pragma unroll
-            for (uint32_t x = LANES; x < 64; x *= 2)
-                d += __shfl_xor(d, x);
-#pragma unroll
-            for (int f = 0; f < 8; ++f) {
-                float a = acc[g][f] * w;
-#pragma unroll
-                for (uint32_t x = LANES; x < 64; x *= 2)
-                    a += __shfl_xor(a, x);
-                acc[g][f] = a;
+            for (int f = 0; f < 4; ++f)
+                acc[g][f] = scatter32(acc[g][f] * w, acc[g][f + 4] * w);
+            if constexpr (ROWS == 4) {
+                acc[g][0] = scatter16(acc[g][0], acc[g][2]);
+                acc[g][1] = scatter16(acc[g][1], acc[g][3]);
             }
             den[g] = d;
             mx[g] = M;
@@ -658,33 +697,48 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         // LDS: acc [W][G][D], then (max, denominator) [W][G][2]
         float* lds_acc = lds;
         float* lds_ml = lds + W * G * D;
-        if (group == 0) {
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float* dst = lds_acc + (wave * G + g) * D;
-                *reinterpret_cast<float4*>(dst + row8::feature(part, 0)) =
+        for (int g = 0; g < G; ++g) {
+            float* dst = lds_acc + (wave * G + g) * D + row8::feature(part, kept);
+            if constexpr (KEEP == 2)
+                *reinterpret_cast<float2*>(dst) = make_float2(acc[g][0], acc[g][1]);
+            else
+                *reinterpret_cast<float4*>(dst) =
                     make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
-                *reinterpret_cast<float4*>(dst + row8::feature(part, 4)) =
-                    make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
-                if (part == 0) {
-                    lds_ml[(wave * G + g) * 2] = mx[g];
-                    lds_ml[(wave * G + g) * 2 + 1] = den[g];
-                }
-            }
+            if (lane == 0)
+                *reinterpret_cast<float2*>(lds_ml + (wave * G + g) * 2) =
+                    make_float2(mx[g], den[g]);
         }
         __syncthreads();
-        // the workgroup's state of q head g, feature f: the W wave states merged
+        // The workgroup's state of q head g, feature f: the W wave states
+        // merged online, four at a time so that their reads are in flight
+        // together (one after another they took half of a microsecond).
         auto wg_state = [&](uint32_t g, uint32_t f, float& M, float& d, float& a) {
             M = -INFINITY;
-            for (uint32_t w = 0; w < W; ++w)
-                M = fmaxf(M, lds_ml[(w * G + g) * 2]);
             d = 0.0f;
             a = 0.0f;
-            for (uint32_t w = 0; w < W; ++w) {
-                const float mw = lds_ml[(w * G + g) * 2];
-                const float weight = mw == -INFINITY ? 0.0f : fast_exp2(mw - M);
-                d += lds_ml[(w * G + g) * 2 + 1] * weight;
-                a += lds_acc[(w * G + g) * D + f] * weight;
+            for (uint32_t w0 = 0; w0 < W; w0 += 4) {
+                float2 ml[4];
+                float av[4];
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const uint32_t at = min(w0 + i, W - 1) * G + g;
+                    ml[i] = *reinterpret_cast<const float2*>(lds_ml + at * 2);
+                    av[i] = lds_acc[at * D + f];
+                    if (w0 + i >= W)
+                        ml[i].x = -INFINITY;
+                }
+                const float nm = fmaxf(fmaxf(M, fmaxf(ml[0].x, ml[1].x)), fmaxf(ml[2].x, ml[3].x));
+                const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
+                d *= keep;
+                a *= keep;
+                M = nm;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const float weight = ml[i].x == -INFINITY ? 0.0f : fast_exp2(ml[i].x - nm);
+                    d += ml[i].y * weight;
+                    a += av[i] * weight;
+                }
             }
         };
         auto emit = [&](uint32_t g, uint32_t f, uint32_t it, float o) {
@@ -747,31 +801,35 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
             const uint32_t slice = t / (G * D), g = (t / D) % G, f = t % D;
             const float* rec = records + g * RF;
             float M = -INFINITY, d = 0.0f, a = 0.0f;
-            auto fold = [&](float mc, float dc, float ac) {
-                const float nm = fmaxf(M, mc);
-                const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
-                const float take = fast_exp2(mc - nm);
-                d = d * keep + dc * take;
-                a = a * keep + ac * take;
-                M = nm;
-            };
-            uint32_t c = slice;
-            for (; c + 3 * S < n_chunks; c += 4 * S) {
+            // four records per round trip, the ones past the last re-reading it
+            // at weight 0 (a slice's records taken one by one cost a round trip
+            // each: rows cut into up to eight chunks spent 2 us here)
+            for (uint32_t c = slice; c < n_chunks; c += 4 * S) {
                 float mc[4], dc[4], ac[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const float* r = rec + (c + u * S) * record_stride;
-                    mc[u] = agent_load(r);
-                    dc[u] = agent_load(r + 1);
-                    ac[u] = agent_load(r + 4 + f);
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const float* r = rec + min(c + i * S, n_chunks - 1) * record_stride;
+                    mc[i] = agent_load(r);
+                    dc[i] = agent_load(r + 1);
+                    ac[i] = agent_load(r + 4 + f);
                 }
+                float nm = fmaxf(M, mc[0]);
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    fold(mc[u], dc[u], ac[u]);
-            }
-            for (; c < n_chunks; c += S) {
-                const float* r = rec + c * record_stride;
-                fold(agent_load(r), agent_load(r + 1), agent_load(r + 4 + f));
+                for (uint32_t i = 1; i < 4; ++i) {
+                    mc[i] = c + i * S < n_chunks ? mc[i] : -INFINITY;
+                    nm = fmaxf(nm, mc[i]);
+                }
+                const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
+                d *= keep;
+                a *= keep;
+                M = nm;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const bool on = i == 0 || c + i * S < n_chunks;
+                    const float take = on ? fast_exp2(mc[i] - nm) : 0.0f;
+                    d += dc[i] * take;
+                    a += ac[i] * take;
+                }
             }
             if (S == 1) {
                 emit(g, f, 1, a / d);

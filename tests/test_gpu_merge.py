@@ -1,0 +1,57 @@
+"""The decode's merges (a wave's row groups, a workgroup's waves, a cut row's
+records) at every remainder of the four states and records they take at a time."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from tests.gpu_util import approx, assert_close, new_context, new_pool, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 16, 17, 33, 100, 161, 300, 520]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = new_context()
+    yield c
+    c.sync()
+    c.close()
+
+
+@pytest.mark.parametrize("code,dim,group", [(orc.BF16, 128, 2), (orc.F32, 128, 1), (orc.F16, 256, 4)])
+def test_merges_at_every_remainder(ctx, code, dim, group, monkeypatch):
+    """1 to 10 waves per workgroup, rows cut into 1 to 33 records."""
+    H, Hq, rows = 2, 2 * group, len(LENGTHS)
+    rng = orc.Mt64(300 + dim + code)
+    pages = [-(-n // 16) for n in LENGTHS]
+    blocks = sum(pages)
+    flat, offsets = rng.permutation(blocks), np.cumsum([0] + pages[:-1])
+    positions = [n - 1 for n in LENGTHS]
+    geom, n = (1, blocks, 16, H, dim), blocks * 16 * H * dim
+    kc, vc = rng.normal(n, code), rng.normal(n, code)
+    q = rng.normal(rows * Hq * dim, code).reshape(rows, -1)
+    scale = float(np.float32(1 / math.sqrt(dim)))
+    expected = orc.Attention(geom, kc, vc, code, q, code, positions, flat, offsets, pages, Hq, 0,
+                             scale).reference()
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(to_dev(vc, code))
+    qd = to_dev(q, code)
+    for waves in (1, 2, 3, 4, 5, 6, 7, 8, 10):
+        for split in (1, 2, 3, 4, 7, 0):
+            monkeypatch.setenv("CKV_DECODE_WAVES", str(waves))
+            monkeypatch.setenv("CKV_DECODE_SPLIT", str(split))
+            pool.upload(flat, offsets, pages, positions)
+            out = torch.full_like(qd, float("nan"))
+            pool.decode(0, qd, Hq, scale, out)
+            ctx.sync()
+            got = to_host(out, code)
+            if code == orc.F32:  # sums of up to 520 terms in another order
+                assert approx(got, expected, 3e-5, 1.0), (waves, split)
+            else:
+                assert_close(orc.to_f32(got, code), expected, what=f"{waves} waves, split {split}")
+    pool.close()
