@@ -349,6 +349,15 @@ uint32_t shortest_tile_blocks(const std::vector<uint32_t>& tiles)
     return (uint32_t)least;
 }
 
+// The workgroups of 32, 64 and 128 rows the tiles take.
+void count_row_blocks(const std::vector<uint32_t>& tiles, uint32_t (&blocks)[3])
+{
+    std::fill(std::begin(blocks), std::end(blocks), 0u);
+    for (size_t t = 0; t < tiles.size(); t += tile_entry_words)
+        for (uint32_t i = 0; i < 3; ++i)
+            blocks[i] += (tiles[t + 1] + (32u << i) - 1) / (32u << i);
+}
+
 // Words of the fast decode plan in the metadata block: the segments'
 // entries, each row's first partial record, then the cut rows.
 size_t plan_words(const decode_plan_shape& shape, size_t rows)
@@ -1296,6 +1305,7 @@ int ckv_tables_upload(ckv_pool* pool, const uint32_t* block_table, size_t n_entr
     m.tiles = pool->d_meta + s_tiles;
     m.n_tiles = (uint32_t)(tiles.size() / tile_entry_words);
     m.tile_blocks = shortest_tile_blocks(tiles);
+    count_row_blocks(tiles, m.row_blocks);
     adopt_batch(pool, rows, n_entries, slots != nullptr, shared, fusable, with_plan, false);
     return CKV_OK;
 }
@@ -1584,6 +1594,7 @@ int ckv_batch_upload(ckv_pool* pool, const uint32_t* seq, const uint32_t* first_
     m.tiles = d + s_tiles;
     m.n_tiles = (uint32_t)(tiles.size() / tile_entry_words);
     m.tile_blocks = shortest_tile_blocks(tiles);
+    count_row_blocks(tiles, m.row_blocks);
     adopt_batch(pool, rows, pool->seq_max * pool->seq_cap, with_slots != 0, shared, fusable,
                 with_plan, true);
     return CKV_OK;
@@ -1849,8 +1860,8 @@ int attention_impl(ckv_pool* pool, size_t layer, const void* queries, size_t q_h
     if (!pool)
         return CKV_E_INVALID_ARGUMENT;
     // src/tensor/attention.cc:290-309: tiles are used when some run of rows
-    // shares a query tile and head_dim <= 128
-    if (pool->shared_tile && pool->head_dim <= 128)
+    // shares a query tile and head_dim <= 128; here 256-wide heads have tiles too
+    if (pool->shared_tile && (pool->head_dim <= 128 || pool->head_dim == 256))
         return prefill_impl(pool, layer, queries, q_heads, scale, output, rows, gate);
     return decode_impl(pool, layer, queries, q_heads, scale, output, rows, gate);
 }

@@ -56,6 +56,7 @@ struct meta_view {
     uint32_t chunk; // tokens per decode work item, a multiple of 16
     uint32_t n_tiles;
     uint32_t tile_blocks; // 32-key blocks the batch's shortest query tile attends (host side)
+    uint32_t row_blocks[3]; // runs of 32, 64 and 128 rows the tiles fall into (host side)
     uint32_t mean_pages; // pages attended per row, mean over the batch (host side)
     uint32_t n_plan;      // workgroups per kv head of the fast decode (the entries they start at)
     uint32_t n_segments;  // entries of plan
@@ -374,9 +375,9 @@ bool decode_uses_fast_path(const pool_view& p, uint32_t q_heads);
 // Floats per (work item, q head) partial record: [max, denominator, 0, 0, acc[head_dim]].
 uint32_t partial_record_floats(uint32_t head_dim);
 
-// ---- launchers (kernels_prefill.hip, kernels_prefill_f32.hip) -----------------
-// MFMA prefill: head_dim 128, 16-token pages, GQA group 1/2/4/8, 16-byte
-// aligned pools, queries and output; bf16/fp16 products on
+// ---- launchers (kernels_prefill.hip, kernels_prefill_wide.hip, kernels_prefill_f32.hip) ----
+// MFMA prefill: head_dim 128 (16-bit pools: or 256), 16-token pages, GQA group
+// 1/2/4/8, 16-byte aligned pools, queries and output; bf16/fp16 products on
 // v_mfma_f32_32x32x16, f32 ones on v_mfma_f32_32x32x2_f32.
 bool prefill_supported(const pool_view& p, uint32_t q_heads, const void* q, const void* out);
 // How a 16-bit prefill launch runs: workgroup waves (8, or 4 when 8-wave
@@ -395,6 +396,12 @@ hipError_t launch_prefill(hipStream_t s, const pool_view& p, const meta_view& m,
                           const void* q, uint32_t q_heads, float scale, void* out,
                           const void* gate, const prefill_shape_info& plan,
                           prefill_split split);
+// The same for 16-bit pools of 256-wide heads (kernels_prefill_wide.hip).
+prefill_shape_info prefill_wide_plan(const pool_view& p, const meta_view& m, uint32_t q_heads,
+                                     int cu_count, uint32_t min_blocks);
+hipError_t launch_prefill_wide(hipStream_t s, const pool_view& p, const meta_view& m,
+                               uint32_t layer, const void* q, uint32_t q_heads, float scale,
+                               void* out, const void* gate, prefill_split split);
 hipError_t launch_prefill_f32(hipStream_t s, const pool_view& p, const meta_view& m,
                               uint32_t layer, const void* q, uint32_t q_heads, float scale,
                               void* out, const void* gate, prefill_split split);

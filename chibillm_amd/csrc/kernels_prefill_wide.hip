@@ -1,0 +1,581 @@
+// Chunked-prefill causal attention over paged KV of 256-wide heads with MFMA
+// tiles (gfx950), bf16 and fp16. The maths, the operand layouts and the hand-over
+// of split tiles are those of kernels_prefill.hip; what differs follows from the
+// head's width.
+//
+// One workgroup of four waves, one per SIMD with up to 512 registers a lane
+// (an O^T of 256 features by 32 queries alone takes 128, Q^T 64), owns 128 / G
+// rows of a query tile for G <= 4 query heads of one kv head; a GQA group of 8
+// takes two workgroups. Per 32-key block and wave: 16 v_mfma_f32_32x32x16 for
+// S^T = K . Q^T and 32 for O^T += V^T . P^T, because P^T enters as two 16-bit
+// terms, its rounding and what the rounding left. Their sum holds 16 bits of a
+// bf16 probability's significand (22 of an fp16 one's), so the result is as
+// exact as with probabilities in 32 bits, which the decode kernels use for
+// such heads: against 64 bits 1.9e-3 of the output in bf16 as before, all of it
+// the rounding of stored values, where one term gives 2.9e-3. fp16 terms are
+// taken at 2^6 times the probability, which the final division removes: small
+// probabilities keep their low term above fp16's smallest value.
+//
+// With one wave on a SIMD nothing else hides a wait, so K operands are read a
+// block ahead: iteration kb multiplies K(kb), already in registers, while the
+// vector ALU forms the probabilities of block kb - 1 and V(kb - 1) is read;
+// then O^T of block kb - 1 is multiplied while K(kb + 1) is read and the scores
+// of block kb are masked and searched for maxima. K has to be staged one block
+// sooner than V: K and V have four LDS stages each (131 KB, one workgroup per
+// compute unit), iteration kb loads K(kb + 3) and V(kb + 2), and its barrier
+// publishes K(kb + 2) and V(kb).
+#include "ckv_internal.h"
+#include "prefill_records.h"
+#include "prefill_tile.h"
+
+#include <algorithm>
+#include <cstdlib>
+
+namespace ckv {
+namespace {
+
+constexpr uint32_t dim = 256;
+constexpr uint32_t page_tokens = 16;
+constexpr uint32_t block_keys = 32;
+constexpr uint32_t waves = 4;
+constexpr uint32_t n_stages = 4;
+constexpr uint32_t k_steps = dim / 16; // products of a block's S^T
+constexpr uint32_t tiles_o = dim / 32; // accumulators of O^T
+
+// K stage: region ks (1 KiB) holds at 16-byte slot 32g + n features 16ks + 8g
+// .. +7 of LDS row n (physical key key_row(n)), the A operand of step ks.
+constexpr uint32_t k_stage_bytes = k_steps * 1024;
+// V stage: two halves of 128 features, each as kernels_prefill.hip stages a
+// 128-wide head: 8 groups of 4 key rows, 64 bytes after each group.
+constexpr uint32_t vg_bytes = 1024 + 64;
+constexpr uint32_t v_half_bytes = 8 * vg_bytes;
+constexpr uint32_t v_stage_bytes = 2 * v_half_bytes;
+constexpr uint32_t regions = 4; // K regions, and V groups, a wave stages per block
+
+// Scale of fp16 probabilities (log2): with the running maximum up to 2^8 stale
+// they reach 2^14, within fp16's range.
+constexpr float p_scale_f16 = 6.0f;
+
+// The source of masked K and V rows.
+__device__ const uint4 zero_row[32] = {};
+
+template <bool F16>
+__device__ __forceinline__ float word_value(uint32_t w, int e)
+{
+    if constexpr (F16)
+        return half_value<true>(static_cast<uint16_t>(w >> (16 * e)));
+    else
+        return __builtin_bit_cast(float, e ? w & 0xFFFF0000u : w << 16);
+}
+
+__device__ __forceinline__ void wait_all_but(uint32_t loads)
+{
+    if (loads >= 12)
+        __builtin_amdgcn_s_waitcnt(0x0F7C); // vmcnt(12)
+    else if (loads >= 8)
+        __builtin_amdgcn_s_waitcnt(0x0F78);
+    else if (loads >= 4)
+        __builtin_amdgcn_s_waitcnt(0x0F74);
+    else
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+}
+
+// FAR: a layer spans more than 4 GiB, so page offsets take 64 bits.
+template <int G, bool F16, bool FAR>
+__global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
+    pool_view p, meta_view md, uint32_t layer, const uint16_t* __restrict__ q,
+    uint16_t* __restrict__ out, uint32_t q_heads, float c, const uint16_t* __restrict__ gate,
+    prefill_split split_scratch)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t lds[n_stages * (k_stage_bytes + v_stage_bytes)];
+    constexpr uint32_t tile_rows = 32 * waves / G;
+    constexpr uint32_t subs = prefill_tile_rows / tile_rows; // workgroups per (tile, head pass, kv head)
+
+    const uint32_t kv_heads = p.kv_heads;
+    const uint32_t group = q_heads / kv_heads;
+    const uint32_t passes = group / G; // 1, or 2 for groups of 8
+    const uint32_t kvh = blockIdx.x % kv_heads;
+    const uint32_t pass = blockIdx.x / kv_heads % passes;
+    // key ranges vary slowest, as in kernels_prefill.hip
+    const uint32_t n_split = split_scratch.n_split;
+    const uint32_t n_rest = md.n_tiles * subs;
+    const uint32_t rest = blockIdx.x / (kv_heads * passes) % n_rest;
+    const uint32_t part = blockIdx.x / (kv_heads * passes) / n_rest;
+    const uint32_t sub = rest % subs;
+    const uint32_t tile = rest / subs;
+    const uint4 te = *reinterpret_cast<const uint4*>(md.tiles + tile_entry_words * tile);
+    const uint32_t count = te.y;
+    const uint32_t r0 = sub * tile_rows;
+    if (r0 >= count)
+        return;
+    const uint32_t nrows = min(tile_rows, count - r0);
+    const uint32_t row0 = te.x + r0;
+    const uint32_t pos0 = te.z + r0;
+    const uint32_t pos_last = pos0 + nrows - 1;
+    const uint32_t* table = md.table + te.w;
+    const uint32_t n_blocks = pos_last / block_keys + 1;
+    const uint32_t n_parts = prefill_range_count(n_blocks, n_split, split_scratch.min_blocks);
+    if (part >= n_parts)
+        return;
+    uint32_t kb_begin, kb_end;
+    prefill_range_bounds(n_blocks, n_parts, part, kb_begin, kb_end);
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t n = lane & 31, g = lane >> 5;
+    const uint32_t F = p.features;
+    const size_t q_stride = (size_t)q_heads * dim;
+
+    // this wave's q-block: one query head, tile rows 32 * (wave / G) + n
+    const uint32_t rb = wave / G;
+    const uint32_t head = kvh * group + pass * G + wave % G;
+    const uint32_t row = rb * 32 + n;
+    const bool valid = row < nrows;
+    const uint32_t qpos = pos0 + min(row, nrows - 1);
+    const size_t qoff = (size_t)(row0 + min(row, nrows - 1)) * q_stride + (size_t)head * dim;
+    const uint32_t pos_lo = pos0 + rb * 32; // the q-block's first position (scalar)
+
+    // Q^T: features 16ks + 8g .. +7 of query n (lanes past the tile's rows hold its
+    // last row again; their results are not written)
+    u32x4_t qr[k_steps];
+#pragma unroll
+    for (uint32_t ks = 0; ks < k_steps; ++ks)
+        qr[ks] = *reinterpret_cast<const u32x4_t*>(q + qoff + ks * 16 + g * 8);
+
+    // Staging: the wave moves K regions wave, wave + 4, .. (features 16 * region
+    // ..: 128 bytes apart) and V groups wave, wave + 4 of each half (the block's
+    // first and second page), one DMA each.
+    const uint64_t page_bytes = (uint64_t)page_tokens * F * 2;
+    const uint64_t base_elems = layer * p.layer_elems + (uint64_t)kvh * dim;
+    const uint8_t* kbytes = uniform_ptr(reinterpret_cast<const uint8_t*>(
+        static_cast<const uint16_t*>(p.keys) + base_elems));
+    const uint8_t* vbytes = uniform_ptr(reinterpret_cast<const uint8_t*>(
+        static_cast<const uint16_t*>(p.values) + base_elems));
+    const uint8_t* zbytes = reinterpret_cast<const uint8_t*>(zero_row);
+    const uint32_t k_key = key_row(n); // this lane's key in a block, and its bytes into the page
+    const bool k_hi = k_key >= page_tokens;
+    const uint32_t k_feat = 16 * wave + 8 * g;
+    const uint32_t k_off = ((k_key & 15) * F + k_feat) * 2;
+    const uint32_t v_key = 4 * (lane >> 4) + wave; // in either page
+    const uint32_t v_off = (v_key * F + (lane & 15) * 8) * 2;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    auto k_stage = [&](uint32_t kb) { return kb % n_stages * k_stage_bytes; };
+    auto v_stage = [&](uint32_t kb) {
+        return n_stages * k_stage_bytes + kb % n_stages * v_stage_bytes;
+    };
+
+    const uint32_t last_entry = pos_last / page_tokens;
+    using c32 = const __attribute__((address_space(4))) uint32_t;
+    const auto* table_s = (const __attribute__((address_space(4))) uint8_t*)(uintptr_t)table;
+    auto page_of = [&](uint32_t entry) { // a scalar load; past the tile's end, its last page
+        return *(c32*)(table_s + 4 * (uint64_t)min(entry, last_entry));
+    };
+    auto load_k = [&](uint32_t kb, uint32_t pg0, uint32_t pg1) {
+        const uint32_t st = lds_base + k_stage(kb) + wave * 1024;
+        const bool whole = kb * block_keys + block_keys - 1 <= pos_last;
+        if (!FAR && whole) {
+            const uint32_t off = (k_hi ? pg1 : pg0) * (uint32_t)page_bytes + k_off;
+#pragma unroll
+            for (uint32_t r = 0; r < regions; ++r)
+                dma16_s(kbytes + 128 * r, off, st + r * waves * 1024);
+        } else {
+            const uint8_t* src = kbytes + (k_hi ? pg1 : pg0) * page_bytes + k_off;
+            if (kb * block_keys + k_key > pos_last)
+                src = zbytes + k_feat * 2;
+#pragma unroll
+            for (uint32_t r = 0; r < regions; ++r)
+                dma16(src + 128 * r, st + r * waves * 1024);
+        }
+    };
+    auto load_v = [&](uint32_t kb, uint32_t pg0, uint32_t pg1) {
+        const uint32_t key0 = kb * block_keys;
+        const bool whole = key0 + block_keys - 1 <= pos_last;
+#pragma unroll
+        for (uint32_t r = 0; r < regions; ++r) { // half r / 2, the block's page r % 2
+            const uint32_t st = lds_base + v_stage(kb) + (r / 2) * v_half_bytes
+                + (wave + 4 * (r % 2)) * vg_bytes;
+            const uint8_t* pv = vbytes + (r % 2 ? pg1 : pg0) * page_bytes + 256 * (r / 2);
+            if (whole) {
+                dma16_s(pv, v_off, st);
+            } else {
+                const bool live = key0 + page_tokens * (r % 2) + v_key <= pos_last;
+                dma16(live ? pv + v_off : zbytes + (lane & 15) * 16, st);
+            }
+        }
+    };
+
+    f32x16_t o[tiles_o];
+#pragma unroll
+    for (uint32_t mt = 0; mt < tiles_o; ++mt)
+        o[mt] = f32x16_t {};
+    float m = -__builtin_inff(), l = 0.0f;
+    float m_limit = -__builtin_inff();
+    const float rescale_raw = rescale_log2 / c;
+    f32x16_t sp; // scores of the block whose probabilities come next
+    float mx = 0.0f;
+    uint4 ka[k_steps];
+
+    auto read_k = [&](uint32_t kb) {
+        const uint8_t* kl = lds + k_stage(kb) + lane * 16;
+#pragma unroll
+        for (uint32_t ks = 0; ks < k_steps; ++ks)
+            ka[ks] = *reinterpret_cast<const uint4*>(kl + ks * 1024);
+    };
+    const uint32_t vr_off = ((lane & 15) >> 2) * vg_bytes + (lane >> 5) * 512
+        + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    // A operand of O^T's accumulator mt: features 32mt + n, keys 16h + 8g + 0..7
+    auto read_v = [&](uint32_t kb, uint4 (&va)[tiles_o][2]) {
+        uint32_t vaddr = lds_base + v_stage(kb) + vr_off;
+        asm volatile("" : "+v"(vaddr));
+        auto* vb = (__attribute__((address_space(3))) uint8_t*)(uintptr_t)vaddr;
+#pragma unroll
+        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+#pragma unroll
+            for (uint32_t h = 0; h < 2; ++h) {
+                auto* at = vb + (mt / 4) * v_half_bytes + 4 * h * vg_bytes + 64 * (mt % 4);
+                const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) i16x4_t*)at);
+                const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) i16x4_t*)(at + 256));
+                const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+                va[mt][h] = make_uint4(l2.x, l2.y, h2.x, h2.y);
+            }
+    };
+    // the probabilities of sp as two 16-bit terms, and their share of the denominator
+    auto probabilities = [&](uint4 (&hi)[2], uint4 (&lo)[2]) {
+        // a range of the keys may hold none a query attends yet (m = -inf)
+        const float bias = F16 ? p_scale_f16 : 0.0f;
+        const float mc = m == -__builtin_inff() ? 0.0f : __builtin_fmaf(m, c, -bias);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            sp[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sp[r], c, -mc));
+        float q4[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            q4[i] = (sp[4 * i] + sp[4 * i + 1]) + (sp[4 * i + 2] + sp[4 * i + 3]);
+        l += (q4[0] + q4[1]) + (q4[2] + q4[3]);
+        uint32_t wh[8], wl[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            wh[i] = pack2<F16>(sp[2 * i], sp[2 * i + 1]);
+            wl[i] = pack2<F16>(sp[2 * i] - word_value<F16>(wh[i], 0),
+                               sp[2 * i + 1] - word_value<F16>(wh[i], 1));
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            hi[h] = make_uint4(wh[4 * h], wh[4 * h + 1], wh[4 * h + 2], wh[4 * h + 3]);
+            lo[h] = make_uint4(wl[4 * h], wl[4 * h + 1], wl[4 * h + 2], wl[4 * h + 3]);
+        }
+    };
+    auto qk = [&]() {
+        f32x16_t s = {};
+#pragma unroll
+        for (uint32_t ks = 0; ks < k_steps; ++ks)
+            s = mfma<F16>(ka[ks], __builtin_bit_cast(uint4, qr[ks]), s);
+        return s;
+    };
+    auto pv = [&](const uint4 (&va)[tiles_o][2], const uint4 (&hi)[2], const uint4 (&lo)[2]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (uint32_t mt = 0; mt < tiles_o; ++mt)
+                o[mt] = mfma<F16>(va[mt][h], hi[h], o[mt]);
+#pragma unroll
+            for (uint32_t mt = 0; mt < tiles_o; ++mt)
+                o[mt] = mfma<F16>(va[mt][h], lo[h], o[mt]);
+        }
+    };
+    // causal mask and maxima of block kb's scores, which become sp
+    auto stats = [&](uint32_t kb, const f32x16_t& s) {
+        sp = s;
+        const uint32_t key0 = kb * block_keys;
+        if (key0 + block_keys - 1 > pos_lo) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t kpos = key0 + 16 * (r >> 3) + 8 * g + (r & 7);
+                if (kpos > qpos)
+                    sp[r] = -__builtin_inff();
+            }
+        }
+        mx = lane_max(sp);
+        return __any(mx > m_limit);
+    };
+    auto rescale = [&]() {
+        const float m_new = fmaxf(m, pair_max(mx));
+        const float alpha = m_new == -__builtin_inff()
+            ? 1.0f
+            : __builtin_amdgcn_exp2f((m - m_new) * c); // 0 at the start
+        l *= alpha;
+        m = m_new;
+        m_limit = m_new + rescale_raw;
+#pragma unroll
+        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+            o[mt] *= alpha;
+    };
+
+    // Before the loop: blocks b .. b + 3 of K and b .. b + 2 of V, those that
+    // the first two iterations read first.
+    uint32_t pk0, pk1, pw0, pw1; // pages of the block whose K, and V, is loaded next
+    {
+        const uint32_t b = kb_begin;
+        uint32_t pg[4][2];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            pg[i][0] = page_of(2 * (b + i));
+            pg[i][1] = page_of(2 * (b + i) + 1);
+        }
+        auto first_k = [&](uint32_t i) {
+            if (b + i < kb_end)
+                load_k(b + i, pg[i][0], pg[i][1]);
+        };
+        auto first_v = [&](uint32_t i) {
+            if (b + i < kb_end)
+                load_v(b + i, pg[i][0], pg[i][1]);
+        };
+        first_k(0);
+        first_k(1);
+        first_v(0);
+        first_k(2);
+        first_v(1);
+        first_k(3);
+        first_v(2);
+        if (b + 3 < kb_end)
+            __builtin_amdgcn_s_waitcnt(0x4F74); // vmcnt(20): K(b) and K(b + 1) have landed
+        else
+            wait_all_but(0);
+        __syncthreads();
+        read_k(b);
+        const f32x16_t s = qk();
+        read_k(min(b + 1, kb_end - 1));
+        stats(b, s);
+        rescale();
+        pk0 = page_of(2 * (b + 4));
+        pk1 = page_of(2 * (b + 4) + 1);
+        pw0 = pg[3][0];
+        pw1 = pg[3][1];
+        wait_all_but(b + 3 < kb_end ? 3 * regions : 0); // K(b + 2) and V(b)
+        __syncthreads();
+    }
+    // K(kb + 3) takes the stage of K(kb - 1), last read (into registers) in
+    // iteration kb - 2, and V(kb + 2) that of V(kb - 2), last read in iteration
+    // kb - 1; a barrier lies between in both cases. The wait leaves in flight
+    // what the wave issued after K(kb + 2): V(kb + 1), K(kb + 3) and V(kb + 2).
+    // Q^T and O^T stay in the accumulation registers (matrix operands may; the
+    // 256 others hold K, V, scores and probabilities): left to itself the
+    // compiler keeps O^T in the others and spills Q^T.
+    auto pin = [&]() {
+#pragma unroll
+        for (uint32_t ks = 0; ks < k_steps; ++ks)
+            asm volatile("" : "+a"(qr[ks]));
+#pragma unroll
+        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+            asm volatile("" : "+a"(o[mt]));
+    };
+    for (uint32_t kb = kb_begin + 1; kb < kb_end; ++kb) {
+        pin();
+        uint32_t newest = kb + 2 < kb_end ? regions : 0;
+        if (kb + 3 < kb_end) {
+            load_k(kb + 3, pk0, pk1);
+            newest += regions;
+        }
+        if (kb + 2 < kb_end) {
+            load_v(kb + 2, pw0, pw1);
+            newest += regions;
+        }
+        uint4 va[tiles_o][2], hi[2], lo[2];
+        read_v(kb - 1, va);
+        const f32x16_t s = qk();   // matrix: block kb
+        probabilities(hi, lo);     // vector: block kb - 1
+        read_k(min(kb + 1, kb_end - 1)); // past the range's end: any staged block
+        pv(va, hi, lo);            // matrix: block kb - 1
+        pw0 = pk0;
+        pw1 = pk1;
+        pk0 = page_of(2 * (kb + 4));
+        pk1 = page_of(2 * (kb + 4) + 1);
+        const bool grew = stats(kb, s); // vector: block kb
+        wait_all_but(newest);
+        __syncthreads();
+        if (grew)
+            rescale();
+    }
+    {
+        uint4 va[tiles_o][2], hi[2], lo[2];
+        read_v(kb_end - 1, va);
+        probabilities(hi, lo);
+        pv(va, hi, lo);
+    }
+
+    float lt = l + __shfl_xor(l, 32); // the query's denominator (both lane halves)
+    if (n_parts > 1) {
+        // The hand-over of kernels_prefill.hip, with 65 chunks of four floats per
+        // (range, query vector): [max, denominator, 0, 0], then acc[4j .. 4j + 3].
+        const uint32_t pair = (rest * passes + pass) * kv_heads + kvh;
+        const uint32_t qv = wave * 32 + n;
+        constexpr uint32_t QV = 32 * waves, chunks = dim / 4 + 1;
+        const __amdgpu_buffer_rsrc_t rs = record_rsrc(
+            split_scratch.records + (uint64_t)pair * n_split * (chunks * QV * 4),
+            n_split * chunks * QV * 16);
+        auto off = [&](uint32_t share, uint32_t chunk) {
+            return ((share * chunks + chunk) * QV + qv) * 16u;
+        };
+#pragma unroll
+        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+#pragma unroll
+            for (uint32_t quad = 0; quad < 4; ++quad)
+                agent_store4(rs, off(part, 1 + 8 * mt + 2 * quad + g), o[mt][4 * quad],
+                             o[mt][4 * quad + 1], o[mt][4 * quad + 2], o[mt][4 * quad + 3]);
+        if (g == 0)
+            agent_store4(rs, off(part, 0), m, lt, 0.0f, 0.0f);
+        wait_vector_memory();
+        __syncthreads(); // also: every wave is past its LDS reads
+        uint32_t* const last_flag = reinterpret_cast<uint32_t*>(lds);
+        if (tid == 0) {
+            const uint32_t before = __hip_atomic_fetch_add(split_scratch.arrivals + pair, 1u,
+                                                           __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t last = before == n_parts - 1;
+            if (last)
+                __hip_atomic_store(split_scratch.arrivals + pair, 0u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            *last_flag = last;
+        }
+        __syncthreads();
+        if (!*last_flag)
+            return;
+        float M = -__builtin_inff();
+        auto weight = [&](float ms, float to) { // 0 for a range that attended nothing
+            return ms == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((ms - to) * c);
+        };
+        lt = 0.0f;
+#pragma unroll
+        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+            o[mt] = f32x16_t {};
+        for (uint32_t s = 0; s < n_parts; ++s) {
+            const u32x4_t hd = agent_load4(rs, off(s, 0));
+            const float ms = __uint_as_float(hd[0]);
+            const float m_new = fmaxf(M, ms);
+            const float keep = weight(M, m_new), w = weight(ms, m_new);
+            M = m_new;
+            lt = lt * keep + __uint_as_float(hd[1]) * w;
+            // a quarter of the range's record at a time (64 registers)
+#pragma unroll
+            for (uint32_t mt = 0; mt < tiles_o; mt += 2) {
+                u32x4_t v[8];
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j)
+                    v[j] = agent_load4(rs, off(s, 1 + 8 * mt + 2 * j + g));
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j)
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) {
+                        const uint32_t r = 4 * (j % 4) + e;
+                        o[mt + j / 4][r] = o[mt + j / 4][r] * keep + __uint_as_float(v[j][e]) * w;
+                    }
+            }
+        }
+    }
+
+    if (!valid)
+        return;
+    const float inv = 1.0f / lt;
+    uint16_t* dst = out + qoff;
+#pragma unroll
+    for (uint32_t mt = 0; mt < tiles_o; ++mt)
+#pragma unroll
+        for (uint32_t quad = 0; quad < 4; ++quad) {
+            const uint32_t f = 32 * mt + 8 * quad + 4 * g;
+            float x[4] = { o[mt][4 * quad] * inv, o[mt][4 * quad + 1] * inv,
+                           o[mt][4 * quad + 2] * inv, o[mt][4 * quad + 3] * inv };
+            if (gate) { // sigmoid_mul (src/qwen/qwen_layer.cc:204) in the epilogue
+                const uint2 gv = *reinterpret_cast<const uint2*>(gate + qoff + f);
+                const uint32_t w[2] = { gv.x, gv.y };
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    x[e] *= sigmoid(half_value<F16>((uint16_t)(w[e / 2] >> (16 * (e % 2)))));
+            }
+            *reinterpret_cast<uint2*>(dst + f) =
+                make_uint2(pack2<F16>(x[0], x[1]), pack2<F16>(x[2], x[3]));
+        }
+}
+
+template <int G>
+hipError_t launch_g(hipStream_t s, const pool_view& p, const meta_view& m, uint32_t layer,
+                    const void* q, uint32_t q_heads, float c, void* out, const void* gate,
+                    uint32_t grid, prefill_split split)
+{
+    const bool far = p.layer_elems * 2 > 0xFFFFFFFFull;
+    const bool f16 = p.dtype == CKV_F16;
+    const auto* qq = static_cast<const uint16_t*>(q);
+    auto* oo = static_cast<uint16_t*>(out);
+    const auto* gg = static_cast<const uint16_t*>(gate);
+    const dim3 blocks(grid), threads(64 * waves);
+    if (f16 && far)
+        prefill_wide_kernel<G, true, true><<<blocks, threads, 0, s>>>(p, m, layer, qq, oo, q_heads, c, gg, split);
+    else if (f16)
+        prefill_wide_kernel<G, true, false><<<blocks, threads, 0, s>>>(p, m, layer, qq, oo, q_heads, c, gg, split);
+    else if (far)
+        prefill_wide_kernel<G, false, true><<<blocks, threads, 0, s>>>(p, m, layer, qq, oo, q_heads, c, gg, split);
+    else
+        prefill_wide_kernel<G, false, false><<<blocks, threads, 0, s>>>(p, m, layer, qq, oo, q_heads, c, gg, split);
+    return hipGetLastError();
+}
+
+// Query heads a workgroup covers of a GQA group, and its rows of a tile.
+uint32_t wide_heads(uint32_t group)
+{
+    return std::min(group, 4u);
+}
+
+} // namespace
+
+// One workgroup per compute unit: if the tiles do not fill them, each tile's
+// keys are split between as many workgroups as do (at most split_max).
+// CKV_PREFILL_SPLIT overrides.
+prefill_shape_info prefill_wide_plan(const pool_view& p, const meta_view& m, uint32_t q_heads,
+                                     int cu_count, uint32_t min_blocks)
+{
+    prefill_shape_info plan { waves, 1, min_blocks, 0, 0 };
+    const uint32_t group = q_heads / p.kv_heads, G = wide_heads(group);
+    // row_blocks[i]: the tiles' workgroups of 32 << i rows
+    const uint64_t busy = (uint64_t)m.row_blocks[G == 4 ? 0 : G == 2 ? 1 : 2] * (group / G) * p.kv_heads;
+    uint64_t split = busy && cu_count > 0 ? (uint64_t)cu_count / busy : 1;
+    if (const char* forced = std::getenv("CKV_PREFILL_SPLIT"))
+        split = (uint64_t)std::max(1L, std::strtol(forced, nullptr, 10));
+    // records are kept for every workgroup of the grid, those past a short
+    // tile's rows included: within 128 MiB
+    const uint64_t grid = (uint64_t)m.n_tiles * (prefill_tile_rows * G / (32 * waves)) * (group / G)
+        * p.kv_heads;
+    const uint64_t floats = grid * (32 * waves) * (dim + 4);
+    const uint64_t room = std::max<uint64_t>(1, ((uint64_t)128 << 20) / sizeof(float) / std::max<uint64_t>(floats, 1));
+    plan.n_split = (uint32_t)std::clamp<uint64_t>(std::min(split, room), 1, split_max);
+    if (plan.n_split > 1) {
+        plan.records_floats = floats * plan.n_split;
+        plan.counters = grid;
+    }
+    return plan;
+}
+
+hipError_t launch_prefill_wide(hipStream_t s, const pool_view& p, const meta_view& m,
+                               uint32_t layer, const void* q, uint32_t q_heads, float scale,
+                               void* out, const void* gate, prefill_split split)
+{
+    const uint32_t group = q_heads / p.kv_heads, G = wide_heads(group);
+    const uint64_t grid = (uint64_t)m.n_tiles * (prefill_tile_rows * G / (32 * waves)) * (group / G)
+        * p.kv_heads * split.n_split;
+    if (!grid)
+        return hipSuccess;
+    if (grid > 0x7FFFFFFFull)
+        return hipErrorInvalidValue;
+    const float c = scale * log2e;
+    switch (G) {
+    case 1:
+        return launch_g<1>(s, p, m, layer, q, q_heads, c, out, gate, (uint32_t)grid, split);
+    case 2:
+        return launch_g<2>(s, p, m, layer, q, q_heads, c, out, gate, (uint32_t)grid, split);
+    default:
+        return launch_g<4>(s, p, m, layer, q, q_heads, c, out, gate, (uint32_t)grid, split);
+    }
+}
+
+} // namespace ckv

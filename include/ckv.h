@@ -301,9 +301,9 @@ int ckv_append_decode(ckv_pool* pool, size_t layer, const void* keys, const void
 /* Prefill form (paged_flash_attention_prefill_f32,
  * src/metal/kernels/attention.metal:246-444): query tiles of consecutive
  * positions of one sequence share every K/V tile; QK^T and PV run on the
- * matrix cores for head_dim 128, 16-token pages, 1, 2, 4 or 8 q heads per kv
- * head and scale > 0 (bf16/fp16 products for 16-bit pools, exact fp32
- * products for f32 pools); other geometries and scales take the decode form
+ * matrix cores for head_dim 128 (16-bit pools: also 256), 16-token pages, 1, 2, 4
+ * or 8 q heads per kv head and scale > 0 (bf16/fp16 products for 16-bit pools,
+ * exact fp32 products for f32 pools); other geometries and scales take the decode form
  * row by row, with the same results. A launch too small to fill the GPU
  * splits each long tile's keys between workgroups and merges their partial states
  * in the pool's scratch (grown on first use, like the decode's split-K

@@ -123,3 +123,76 @@ def test_wide_decode_matches_oracle_and_general_path(ctx, code, group, rotary, g
             assert approx(got, expected, 3e-5, 1.0), what
         else:
             assert_close(orc.to_f32(got, code), expected, what=what)
+
+
+# (prefix, rows) of each sequence: single rows, tile and block edges, tiles of several workgroups
+CHUNKS = [(0, 1), (0, 33), (5, 40), (31, 64), (100, 128), (16, 257), (700, 1), (1000, 70), (63, 2)]
+
+
+@pytest.mark.parametrize("code,group,gated,split,min_blocks", [
+    (orc.BF16, 4, True, None, None), (orc.F16, 4, False, "1", None), (orc.BF16, 2, False, "3", "1"),
+    (orc.F16, 1, True, "8", "2"), (orc.BF16, 8, True, "2", "1"), (orc.F16, 2, True, "8", "1"),
+    (orc.BF16, 1, False, None, None), (orc.F32, 4, True, None, None)])
+def test_wide_prefill_matches_oracle_and_general_path(ctx, code, group, gated, split, min_blocks,
+                                                      monkeypatch):
+    """Tiles on the matrix cores (f32 pools: decode rows) with keys unsplit and
+    split. Probabilities enter as two 16-bit terms, so the error against the
+    double reference is that of the general path, which holds them in 32 bits:
+    both round the same stored values once (bounded at 1.1 times here, for the
+    order of sums)."""
+    print(f"wide prefill dtype {code} group {group} gated {gated} split {split}", flush=True)
+    if split is not None:
+        monkeypatch.setenv("CKV_PREFILL_SPLIT", split)
+    if min_blocks is not None:
+        monkeypatch.setenv("CKV_PREFILL_SPLIT_MIN", min_blocks)
+    rng = orc.Mt64(1200 + 10 * group + code)
+    H = 2
+    Hq, F = H * group, H * D
+    spans = [p + n for p, n in CHUNKS]
+    pages = [-(-n // 16) for n in spans]
+    blocks = sum(pages) + 2
+    order = rng.permutation(blocks)
+    tables = np.split(order[:sum(pages)], np.cumsum(pages)[:-1])
+    flat, starts = np.concatenate(tables), np.cumsum([0] + pages[:-1])
+    seq = np.repeat(np.arange(len(CHUNKS)), [n for _, n in CHUNKS])
+    positions = np.concatenate([np.arange(p, p + n) for p, n in CHUNKS]).astype(np.uint32)
+    offsets, lengths = starts[seq], np.array(pages)[seq]
+    rows, geom = len(positions), (1, blocks, 16, H, D)
+    kc, vc = nan_pages(code, blocks * 16 * F), nan_pages(code, blocks * 16 * F)
+    for t, n in zip(tables, spans):
+        orc.store_kv(kc, vc, rng.normal(n * F, code).reshape(-1, F),
+                     rng.normal(n * F, code).reshape(-1, F), [orc.slot(t, p, 16) for p in range(n)],
+                     0, blocks * 16)
+    q = rng.normal(rows * Hq * D, code).reshape(rows, -1)
+    gate = rng.normal(rows * Hq * D, code).reshape(rows, -1) if gated else None
+    scale = float(np.float32(1 / math.sqrt(D)))
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(to_dev(vc, code))
+    pool.upload(flat, offsets, lengths, positions)
+    gd = to_dev(gate, code) if gated else None
+    outs = []
+    for shift in (lambda t: t, lambda t: t, misaligned):
+        qd = shift(to_dev(q, code))
+        out = shift(torch.full((rows, Hq * D), float("nan"), dtype=qd.dtype, device="cuda"))
+        if gated:
+            pool.attention_gated(0, qd, Hq, scale, gd, out)
+        else:
+            pool.attention(0, qd, Hq, scale, out)
+        ctx.sync()
+        outs.append(to_host(out, code))
+    pool.close()
+    assert np.array_equal(outs[0], outs[1]), "a second call differs"
+    expected = orc.Attention(geom, kc, vc, code, q, code, positions, flat, offsets, lengths, Hq, 0,
+                             scale).reference()
+    if gated:
+        g = gate if code == orc.F32 else orc.to_f32(gate, code)
+        expected = expected * (1.0 / (1.0 + np.exp(-np.asarray(g, np.float64))))
+    got, general = ((x if code == orc.F32 else orc.to_f32(x, code)).astype(np.float64)
+                    for x in (outs[0], outs[2]))
+    if code == orc.F32:
+        assert approx(got, expected, 3e-5, 1.0)
+    else:
+        assert_close(got, expected, what="prefill")
+        off, off_general = (np.linalg.norm(x - expected) for x in (got, general))
+        assert off <= 1.1 * off_general, (off, off_general)
