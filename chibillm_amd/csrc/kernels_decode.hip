@@ -22,10 +22,12 @@
 // Generic path (any head_dim <= 1024, any page size): split-KV over token
 // chunks, one wave per (chunk, kv_head), and a merge launch.
 #include "ckv_internal.h"
+#include "prefill_records.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 namespace ckv {
 namespace {
@@ -34,8 +36,6 @@ constexpr float log2e = 1.4426950408889634f;
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 // K/V pages are read once per decode step: nontemporal loads stream them
 // past the caches (measured on MI355X: plain 16-byte streaming reads top out
@@ -103,11 +103,11 @@ __device__ __forceinline__ float fast_exp2(float x)
 // records, count themselves in, and the last to arrive merges) is a protocol
 // of this target's memory system, not a release/acquire pair of the HIP
 // memory model:
-//   - records are written with relaxed agent-scope atomic stores and read
-//     with relaxed agent-scope atomic loads; on gfx950 (the GFX942 rows of
-//     LLVM's AMDGPU memory model) these are global_store/global_load with sc1,
-//     which write through and bypass any L2 line that could be stale, so
-//     every XCD sees them in memory without an L2 writeback;
+//   - records are written and read 16 bytes at a time with the sc1 cache policy
+//     (prefill_records.h): what relaxed agent-scope atomic accesses carry on
+//     gfx950 (the GFX942 rows of LLVM's AMDGPU memory model), which write
+//     through and bypass any L2 line that could be stale, so every XCD sees
+//     them in memory without an L2 writeback;
 //   - each writer waits with s_waitcnt vmcnt(0) for its stores to complete
 //     (on GFX9-family parts vmcnt counts stores too) before one thread's
 //     relaxed agent-scope fetch-add counts the chunk in; the last arriver's
@@ -121,27 +121,6 @@ __device__ __forceinline__ float fast_exp2(float x)
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "kernels_decode.hip's split-K handoff relies on gfx950's memory system; build for gfx950"
 #endif
-
-// Relaxed agent-scope accesses: coherent across the XCDs on their own (the
-// store writes through, the load misses any cache line that could be stale),
-// so data passed this way between workgroups needs no L2 writeback, only
-// the writer's wait for its stores to complete before it signals.
-__device__ __forceinline__ void agent_store(float* p, float v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ float agent_load(const float* p)
-{
-    return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Waits until every vector memory access this wave issued (stores included)
-// has completed; a compiler barrier too.
-__device__ __forceinline__ void wait_vector_memory()
-{
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
 
 // f32 -> bf16 round to nearest even, NaN quieted (src/tensor/types.h:60-75).
 __device__ __forceinline__ uint32_t bf16_bits(float x)
@@ -356,6 +335,39 @@ __device__ __forceinline__ float load_elem(const void* base, uint64_t i)
         return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<const uint16_t*>(base)[i]));
 }
 
+// Four consecutive elements, 4-element aligned.
+template <int DT>
+__device__ __forceinline__ void load4(const void* base, uint64_t i, float (&x)[4])
+{
+    if constexpr (DT == CKV_F32) {
+        const float4 v = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
+        x[0] = v.x;
+        x[1] = v.y;
+        x[2] = v.z;
+        x[3] = v.w;
+    } else {
+        using ops = half2_ops<DT == CKV_F16>;
+        const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + i);
+        x[0] = ops::lo(v.x);
+        x[1] = ops::hi(v.x);
+        x[2] = ops::lo(v.y);
+        x[3] = ops::hi(v.y);
+    }
+}
+
+template <int DT>
+__device__ __forceinline__ void store4(void* base, uint64_t i, const float (&x)[4])
+{
+    if constexpr (DT == CKV_F32) {
+        *reinterpret_cast<float4*>(static_cast<float*>(base) + i) =
+            make_float4(x[0], x[1], x[2], x[3]);
+    } else {
+        using ops = half2_ops<DT == CKV_F16>;
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(base) + i) =
+            make_uint2(ops::pack(x[0], x[1]), ops::pack(x[2], x[3]));
+    }
+}
+
 template <int DT>
 __device__ __forceinline__ void store_elem(void* base, uint64_t i, float x)
 {
@@ -429,6 +441,9 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
     // them now, beside the plan entry, not after it
     asm volatile("" ::"s"(kl), "s"(vl), "s"(m.table), "s"(row_bytes), "s"(q));
 
+    // a gate aligned for vector loads (only the pool, queries and output need be)
+    const bool gate_vectors = GATED && (reinterpret_cast<uintptr_t>(gate) & (4 * ES - 1)) == 0;
+
     // One segment: pages [pg_first, pg_end) of a row, chunk `chunk` of the
     // row's n_chunks (e0 = row, chunk, the row's position, the flat table
     // index of page pg_first; e1 = pg_first, pg_end, n_chunks, next entry).
@@ -449,11 +464,6 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         const uint32_t pg_first = e1.x;
         const uint32_t u_end = UPP == 1 ? e1.y : min(e1.y * UPP, u_last + 1);
         const uint32_t n_chunks = e1.z;
-        float gate_early = 0.0f; // the first epilogue iteration's gate value (one register)
-        if constexpr (GATED) {
-            if (tid < G * D)
-                gate_early = load_elem<DT>(gate, ((uint64_t)row * q_heads + qh0) * D + tid);
-        }
         const uint32_t* tbl = m.table + (e0.w - pg_first); // the row's table
 
         row8 qv[G];
@@ -661,13 +671,32 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         }
         __builtin_amdgcn_s_setprio(0); // the merge at the default priority
 
+        // Four features of the workgroup's result per thread from here on
+        constexpr uint32_t T4 = G * D / 4;
+        const uint64_t out_row = ((uint64_t)row * q_heads + qh0) * D;
+        // the gate's values, loaded now so that their latency hides behind the
+        // merge (the pages' registers are free)
+        float gate4[4];
+        auto load_gate = [&](uint32_t t) {
+            if (gate_vectors) {
+                load4<DT>(gate, out_row + 4 * t, gate4);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    gate4[e] = load_elem<DT>(gate, out_row + 4 * t + e);
+            }
+        };
+        if constexpr (GATED)
+            if (tid < T4)
+                load_gate(tid);
+
         // What follows bounds small batches: a launch over six rows of up to
         // 1,500 tokens has its last page scored after 5.5 us and ended at
         // 10.9, waiting on one LDS or memory round trip after another. With
-        // the swaps below and the reads of the merges four at a time a layer
-        // of that batch takes 11.5 us instead of 12.9, four rows of U[64, 512]
-        // 9.3 instead of 10.4, one 32K row 30.3 instead of 31.4 (launch gaps
-        // included, rotated).
+        // the swaps below, the reads of the merges four at a time and 16 bytes
+        // per access a layer of that batch takes 11.6 us instead of 12.9, four
+        // rows of U[64, 512] 9.0 instead of 10.4, one 32K row 29.7 instead of
+        // 31.3 (launch gaps included, rotated).
         // Merge the wave's row-group states. The maxima and denominators are
         // reduced into every lane; the accumulators are reduced and scattered,
         // each swap halving what a lane holds: of its features 0..7 a lane of
@@ -710,77 +739,93 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                     make_float2(mx[g], den[g]);
         }
         __syncthreads();
-        // The workgroup's state of q head g, feature f: the W wave states
-        // merged online, four at a time so that their reads are in flight
-        // together (one after another they took half of a microsecond).
-        auto wg_state = [&](uint32_t g, uint32_t f, float& M, float& d, float& a) {
+        // The workgroup's state of q head g, features f .. f + 3: the n states in
+        // LDS (the waves', or the slices' below) merged online, four at a time
+        // so that their reads are in flight together (one after another they
+        // took half a microsecond).
+        auto wg_state = [&](uint32_t n, uint32_t g, uint32_t f, float& M, float& d, float (&a)[4]) {
             M = -INFINITY;
             d = 0.0f;
-            a = 0.0f;
-            for (uint32_t w0 = 0; w0 < W; w0 += 4) {
+            a[0] = a[1] = a[2] = a[3] = 0.0f;
+            for (uint32_t w0 = 0; w0 < n; w0 += 4) {
                 float2 ml[4];
-                float av[4];
+                float4 av[4];
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i) {
-                    const uint32_t at = min(w0 + i, W - 1) * G + g;
+                    const uint32_t at = min(w0 + i, n - 1) * G + g;
                     ml[i] = *reinterpret_cast<const float2*>(lds_ml + at * 2);
-                    av[i] = lds_acc[at * D + f];
-                    if (w0 + i >= W)
+                    av[i] = *reinterpret_cast<const float4*>(lds_acc + at * D + f);
+                    if (w0 + i >= n)
                         ml[i].x = -INFINITY;
                 }
                 const float nm = fmaxf(fmaxf(M, fmaxf(ml[0].x, ml[1].x)), fmaxf(ml[2].x, ml[3].x));
                 const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
                 d *= keep;
-                a *= keep;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    a[e] *= keep;
                 M = nm;
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i) {
                     const float weight = ml[i].x == -INFINITY ? 0.0f : fast_exp2(ml[i].x - nm);
                     d += ml[i].y * weight;
-                    a += av[i] * weight;
+                    a[0] += av[i].x * weight;
+                    a[1] += av[i].y * weight;
+                    a[2] += av[i].z * weight;
+                    a[3] += av[i].w * weight;
                 }
             }
         };
-        auto emit = [&](uint32_t g, uint32_t f, uint32_t it, float o) {
-            const uint64_t at = ((uint64_t)row * q_heads + qh0 + g) * D + f;
-            if constexpr (GATED)
-                o *= sigmoid(it == 0 ? gate_early : load_elem<DT>(gate, at));
-            store_elem<DT>(out, at, o);
+        // thread t's four features, divided by the denominator, gated, rounded once
+        auto emit = [&](uint32_t t, const float (&a)[4], float d) {
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                o[e] = a[e] / d;
+            if constexpr (GATED) {
+                if (t != tid)
+                    load_gate(t);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[e] *= sigmoid(gate4[e]);
+            }
+            store4<DT>(out, out_row + 4 * t, o);
         };
         if (n_chunks == 1) {
-            uint32_t it = 0;
-            for (uint32_t t = tid; t < G * D; t += blockDim.x, ++it) {
-                float M, d, a;
-                wg_state(t / D, t % D, M, d, a);
-                emit(t / D, t % D, it, a / d);
+            for (uint32_t t = tid; t < T4; t += blockDim.x) {
+                float M, d, a[4];
+                wg_state(W, t / (D / 4), 4 * t % D, M, d, a);
+                emit(t, a, d);
             }
             return;
         }
         // a chunk of a cut row: record [max, denominator, 0, 0, acc[D]] per q head,
-        // stored at agent scope (through to where every XCD reads it)
+        // stored through to where every XCD reads it, 16 bytes per thread
         constexpr uint32_t RF = D + 4;
-        const uint64_t record_stride = (uint64_t)q_heads * RF; // between a row's chunks
+        const uint32_t record_stride = q_heads * RF; // between a row's chunks, in floats
         float* const records = split.records
             + ((uint64_t)m.split_first[row] * q_heads + qh0) * RF;
-        for (uint32_t t = tid; t < G * D; t += blockDim.x) {
-            const uint32_t g = t / D, f = t % D;
-            float M, d, a;
-            wg_state(g, f, M, d, a);
-            float* rec = records + chunk * record_stride + g * RF;
-            agent_store(rec + 4 + f, a);
-            if (f == 0) {
-                agent_store(rec, M);
-                agent_store(rec + 1, d);
+        {
+            const __amdgpu_buffer_rsrc_t rec =
+                record_rsrc(records + (uint64_t)chunk * record_stride, G * RF * 4);
+            for (uint32_t t = tid; t < T4; t += blockDim.x) {
+                const uint32_t g = t / (D / 4), f = 4 * t % D;
+                float M, d, a[4];
+                wg_state(W, g, f, M, d, a);
+                agent_store4(rec, (g * RF + 4 + f) * 4, a[0], a[1], a[2], a[3]);
+                if (f == 0)
+                    agent_store4(rec, g * RF * 4, M, d, 0.0f, 0.0f);
             }
         }
         // Arrival: every wave waits until its record stores are complete, then
         // one thread counts the chunk in. The chunk that arrives last resets the
-        // counter and merges the row's records (agent-scope loads, so none comes
-        // from a stale cache line); the others are done.
+        // counter and merges the row's records (their loads miss any cache line
+        // that could be stale); the others are done.
         wait_vector_memory();
         __syncthreads();
         uint32_t* const arrivals = split.arrivals + (uint64_t)m.split_first[row] * H + kv_head;
-        uint32_t* const last_flag = reinterpret_cast<uint32_t*>(lds_ml); // lds_ml is read out
+        uint32_t* const last_flag =
+            reinterpret_cast<uint32_t*>(lds_ml + W * G * 2 + (ROPE ? rotary : 0));
         if (tid == 0) {
             const uint32_t before =
                 __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -794,70 +839,72 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
             return;
         // Thread (slice, g, f) folds chunks slice, slice + S, ... of q head g with
         // weights 2^(m_c - M) (paged_attention_reduce_f32,
-        // src/metal/kernels/attention.metal:567-615, done online); the S slices are
-        // folded through LDS and the result normalised, gated and rounded once.
-        const uint32_t S = blockDim.x >= G * D ? blockDim.x / (G * D) : 1;
-        for (uint32_t t = tid; t < S * G * D; t += blockDim.x) {
-            const uint32_t slice = t / (G * D), g = (t / D) % G, f = t % D;
-            const float* rec = records + g * RF;
-            float M = -INFINITY, d = 0.0f, a = 0.0f;
-            // four records per round trip, the ones past the last re-reading it
-            // at weight 0 (a slice's records taken one by one cost a round trip
-            // each: rows cut into up to eight chunks spent 2 us here)
-            for (uint32_t c = slice; c < n_chunks; c += 4 * S) {
-                float mc[4], dc[4], ac[4];
+        // src/metal/kernels/attention.metal:567-615, done online), as many
+        // records per round trip as a slice has, up to four; the S slices are
+        // folded through LDS. The loads go to memory, past the caches: a record
+        // past the row's last is not read.
+        // (slices enough for four records each; W of them fit the wave states' LDS)
+        const uint32_t S = max(1u, min(min(blockDim.x / T4, W), (n_chunks + 3) / 4));
+        auto fold = [&](auto width) {
+            constexpr uint32_t U = decltype(width)::value;
+            for (uint32_t t = tid; t < S * T4; t += blockDim.x) {
+                const uint32_t slice = t / T4, g = t % T4 / (D / 4), f = 4 * t % D;
+                float M = -INFINITY, d = 0.0f, a[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+                for (uint32_t c0 = 0; c0 < n_chunks; c0 += U * S) {
+                    const uint32_t left = n_chunks - c0; // records from here
+                    const __amdgpu_buffer_rsrc_t rec =
+                        record_rsrc(records + (uint64_t)c0 * record_stride,
+                                    (min(left, U * S) - 1) * record_stride * 4 + G * RF * 4);
+                    u32x4_t head[U], part4[U];
 #pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) {
-                    const float* r = rec + min(c + i * S, n_chunks - 1) * record_stride;
-                    mc[i] = agent_load(r);
-                    dc[i] = agent_load(r + 1);
-                    ac[i] = agent_load(r + 4 + f);
-                }
-                float nm = fmaxf(M, mc[0]);
+                    for (uint32_t i = 0; i < U; ++i) {
+                        // out of the descriptor's range for a record past the last: reads 0
+                        const uint32_t at = ((slice + i * S) * record_stride + g * RF) * 4;
+                        head[i] = agent_load4(rec, at);
+                        part4[i] = agent_load4(rec, at + (4 + f) * 4);
+                    }
+                    float mc[U], nm = M;
 #pragma unroll
-                for (uint32_t i = 1; i < 4; ++i) {
-                    mc[i] = c + i * S < n_chunks ? mc[i] : -INFINITY;
-                    nm = fmaxf(nm, mc[i]);
-                }
-                const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
-                d *= keep;
-                a *= keep;
-                M = nm;
+                    for (uint32_t i = 0; i < U; ++i) {
+                        mc[i] = slice + i * S < left ? __uint_as_float(head[i][0]) : -INFINITY;
+                        nm = fmaxf(nm, mc[i]);
+                    }
+                    const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
+                    d *= keep;
 #pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) {
-                    const bool on = i == 0 || c + i * S < n_chunks;
-                    const float take = on ? fast_exp2(mc[i] - nm) : 0.0f;
-                    d += dc[i] * take;
-                    a += ac[i] * take;
+                    for (int e = 0; e < 4; ++e)
+                        a[e] *= keep;
+                    M = nm;
+#pragma unroll
+                    for (uint32_t i = 0; i < U; ++i) {
+                        const float take = slice + i * S < left ? fast_exp2(mc[i] - nm) : 0.0f;
+                        d += __uint_as_float(head[i][1]) * take;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            a[e] += __uint_as_float(part4[i][e]) * take;
+                    }
                 }
+                if (S == 1) {
+                    emit(t, a, d);
+                    continue;
+                }
+                *reinterpret_cast<float4*>(lds_acc + (slice * G + g) * D + f) =
+                    make_float4(a[0], a[1], a[2], a[3]);
+                if (f == 0)
+                    *reinterpret_cast<float2*>(lds_ml + (slice * G + g) * 2) = make_float2(M, d);
             }
-            if (S == 1) {
-                emit(g, f, 1, a / d);
-                continue;
-            }
-            lds_acc[(slice * G + g) * D + f] = a;
-            if (f == 0) {
-                lds_ml[2 + (slice * G + g) * 2] = M;
-                lds_ml[2 + (slice * G + g) * 2 + 1] = d;
-            }
-        }
+        };
+        if (n_chunks <= 2 * S)
+            fold(std::integral_constant<uint32_t, 2> {});
+        else
+            fold(std::integral_constant<uint32_t, 4> {});
         if (S == 1)
             return;
         __syncthreads();
-        for (uint32_t t = tid; t < G * D; t += blockDim.x) {
-            const uint32_t g = t / D, f = t % D;
-            float M = -INFINITY;
-            for (uint32_t sl = 0; sl < S; ++sl)
-                M = fmaxf(M, lds_ml[2 + (sl * G + g) * 2]);
-            float d = 0.0f, a = 0.0f;
-            for (uint32_t sl = 0; sl < S; ++sl) {
-                const float ms = lds_ml[2 + (sl * G + g) * 2];
-                // a slice may hold no chunk
-                const float w = ms == -INFINITY ? 0.0f : fast_exp2(ms - M);
-                d += lds_ml[2 + (sl * G + g) * 2 + 1] * w;
-                a += lds_acc[(sl * G + g) * D + f] * w;
-            }
-            emit(g, f, 1, a / d);
+        for (uint32_t t = tid; t < T4; t += blockDim.x) {
+            float M, d, a[4];
+            wg_state(S, t / (D / 4), 4 * t % D, M, d, a);
+            emit(t, a, d);
         }
     };
 
@@ -1126,8 +1173,8 @@ hipError_t launch_fast(hipStream_t s, const pool_view& p, const meta_view& m, ui
     const uint32_t units = m.n_plan * p.kv_heads;
     const uint32_t waves = fast_waves(G, dt, units, cu_count, m.mean_pages, m.split_pages);
     const dim3 grid(units), block(64 * waves);
-    // the merge's (acc, max, denominator) per wave, then the rope angle table
-    const size_t lds = ((size_t)waves * G * (D + 2) + (rope ? rotary : 0)) * sizeof(float);
+    // the merge's (acc, max, denominator) per wave, the rope angle table, a flag
+    const size_t lds = ((size_t)waves * G * (D + 2) + (rope ? rotary : 0) + 1) * sizeof(float);
     const auto qq = static_cast<const char*>(q);
     const auto ki = static_cast<const char*>(k_in);
     const auto vi = static_cast<const char*>(v_in);
