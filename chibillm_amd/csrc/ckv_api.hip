@@ -393,7 +393,8 @@ int ensure_plan(ckv_pool* pool)
         return CKV_OK;
     ckv_context* ctx = pool->ctx;
     const decode_plan_shape shape = shape_decode_plan(
-        pool->positions, (uint32_t)pool->block_size, (uint32_t)pool->kv_heads, ctx->cu_count);
+        pool->positions, (uint32_t)pool->block_size, (uint32_t)pool->kv_heads, ctx->cu_count,
+        decode_form_of(pool->dtype, (uint32_t)pool->head_dim));
     const size_t words = std::max<size_t>(plan_words(shape, pool->positions.size()), 4);
     void* host = nullptr;
     int status = stage(ctx, words * sizeof(uint32_t), &host);
@@ -1259,7 +1260,8 @@ int ckv_tables_upload(ckv_pool* pool, const uint32_t* block_table, size_t n_entr
     // up now
     const bool with_plan = !shared;
     const decode_plan_shape plan_shape = with_plan
-        ? shape_decode_plan(pool->positions, (uint32_t)bs, (uint32_t)pool->kv_heads, ctx->cu_count)
+        ? shape_decode_plan(pool->positions, (uint32_t)bs, (uint32_t)pool->kv_heads, ctx->cu_count,
+        decode_form_of(pool->dtype, (uint32_t)pool->head_dim))
         : decode_plan_shape {};
 
     // pack: table | offsets | lengths | positions | slots | tiles | plan
@@ -1514,7 +1516,8 @@ int ckv_batch_upload(ckv_pool* pool, const uint32_t* seq, const uint32_t* first_
         }
     const bool with_plan = !shared;
     const decode_plan_shape plan_shape = with_plan
-        ? shape_decode_plan(positions, (uint32_t)bs, (uint32_t)pool->kv_heads, ctx->cu_count)
+        ? shape_decode_plan(positions, (uint32_t)bs, (uint32_t)pool->kv_heads, ctx->cu_count,
+        decode_form_of(pool->dtype, (uint32_t)pool->head_dim))
         : decode_plan_shape {};
 
     // d_meta: offsets | lengths | positions | slots (written by the expand

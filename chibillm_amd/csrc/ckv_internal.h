@@ -330,8 +330,17 @@ struct decode_plan_shape {
     uint64_t deal_work;   // balanced: the work dealt out (pages and segment costs)
     bool balanced;
 };
+struct decode_form {
+    uint32_t per_cu;      // workgroups a compute unit holds
+    uint32_t min_pages;   // shortest chunk cut, but for the rest of a row
+    uint32_t max_chunks;  // most chunks of a row
+    uint32_t uncut_slack; // pages by which a row may exceed the share and stay whole
+    bool few_waves;       // workgroups too small to read a whole row at full rate
+};
+decode_form decode_form_of(int dtype, uint32_t head_dim);
 decode_plan_shape shape_decode_plan(const std::vector<uint32_t>& positions, uint32_t block_size,
-                                    uint32_t kv_heads, int cu_count);
+                                    uint32_t kv_heads, int cu_count,
+                                    const decode_form& form = decode_form_of(CKV_BF16, 128));
 // Waves per workgroup of the fast decode for a launch of `units` (plan
 // workgroup, kv head) workgroups: a plan's split_pages (0 when no row is cut)
 // and the batch's mean row pages decide it; CKV_DECODE_WAVES overrides.

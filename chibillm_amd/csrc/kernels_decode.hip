@@ -939,30 +939,21 @@ __device__ __forceinline__ float wave_sum(float v)
 constexpr int generic_max_features_per_lane = 16; // head_dim <= 1024
 
 // Cut rows (shape_decode_plan). The balanced plan deals the batch's pages to
-// split_wgs_per_cu workgroups of split_waves waves per compute unit (all of
-// them resident at once), with a segment costing split_segment_pages pages
-// and no piece shorter than split_min_piece; no more workgroups than rows
-// where pieces would fall under split_min_pages, and no row in more than
-// split_max_chunks pieces (the merge of a row reads its pieces' records:
-// measured on MI355X, a 32K-token row cut into 128 chunks of 16 pages
-// decodes in 24 us and merges in 7.5 us, in 32 chunks of 64 pages the pair
-// takes 29 us in all). With more rows than workgroups, or under
-// split_balance_min_pages pages per workgroup, the round trips of the
-// segments a workgroup runs one after another cost more than the balance
-// gains, and rows are cut into fixed chunks of a quarter of a compute unit's
-// share instead (the config-5 churn took 3 % longer dealing its batches of
-// hundreds of rows).
-// Measured on one MI355X layer (bf16, 8 kv heads, fused append + decode,
-// against fixed chunks throughout): batch 32 of U[256, 4096] tokens -2.8 %
-// time (-0.7 % unfused), 32 rows of 1,024 tokens -14 %, of 4,096 -1.3 %,
-// 64 rows of U[64, 2048] and one 32K-token row within 0.6 %.
-constexpr uint64_t split_wgs_per_cu = 2;
-constexpr uint64_t split_min_pages = 12;
+// as many workgroups as the GPU holds at once (decode_form::per_cu per compute
+// unit), with a segment costing split_segment_pages pages and no piece shorter
+// than split_min_piece; no more workgroups than rows where pieces would fall
+// under the form's min_pages, and no row in more than max_chunks pieces (the
+// merge of a row reads its pieces' records). With more rows than workgroups the
+// round trips of the segments a workgroup runs one after another cost more than
+// the balance gains, and rows are cut into fixed chunks of a quarter of a
+// compute unit's share instead (the config-5 churn took 3 % longer dealing its
+// batches of hundreds of rows); batches of under split_balance_min_pages pages
+// per workgroup, and all of 256-wide heads, weigh the two (small_batch_span).
+constexpr uint64_t split_row_pages = 10;
 constexpr uint64_t split_min_piece = 4;
 constexpr uint64_t split_balance_min_pages = 32;
 constexpr uint64_t split_per_share = 4;
 constexpr uint64_t split_segment_pages = 4;
-constexpr uint64_t split_max_chunks = 32;
 constexpr uint32_t split_waves = 8;
 // Waves per workgroup of a cut plan whose workgroups fit one per compute unit
 // and hold at least split_alone_min_pages pages each (one long row's pieces):
@@ -974,14 +965,26 @@ constexpr uint32_t split_waves_alone = 12;
 constexpr uint32_t split_alone_min_pages = 48;
 // Pages (about 12 us of one workgroup's reads) by which the longest row may
 // exceed 9/8 of a compute unit's share and still stay whole, for batches of
-// one or two (row, kv head) units per compute unit. Measured on one
+// one or two (row, kv head) units per compute unit (and no more than 13/8 of
+// the share: 32 rows of U[300, 2000] tokens, longest 1.73 times the share, cut
+// 31.7 us, whole 34.5). Measured on one
 // MI355X layer (fused, bf16, 8 kv heads) against cutting: 32 rows of
 // U[512, 1536] tokens -15 %, U[768, 1280] -9 %, 1,024 tokens -7 %, 2,048 -6 %,
 // 64 rows of U[64, 2048] -5 %, 48 rows of U[256, 4096] -3.5 %; config 2's 32
 // rows of U[256, 4096] (longest 256 pages, share 144) still cut, as do batches
 // of fewer (row, kv head) units than compute units (8 rows of 1,024 tokens
 // whole: +36 %).
-constexpr uint64_t split_uncut_slack = 47;
+constexpr uint32_t split_uncut_slack = 47;
+// How a pool's decode fills the GPU (decode_form). 16-bit pages of 128-wide
+// heads: two 8-wave workgroups per compute unit. f32 pages: two of 4 waves; a
+// whole row on 4 waves reads at a fraction of a compute unit's rate, so rows are
+// not kept whole for want of balance alone (48 rows of U[256, 4096] tokens whole
+// 170 us, dealt out 130). 256-wide heads: one workgroup of 8 waves (with more
+// than two q heads per kv head its lanes need the registers of two); a page is
+// twice the bytes, so chunks may be shorter and the slack is half.
+constexpr decode_form form_narrow { 2, 12, 32, split_uncut_slack, false };
+constexpr decode_form form_f32 { 2, 8, 32, 0, true };
+constexpr decode_form form_wide { 1, 4, 128, split_uncut_slack / 2, false };
 
 // One wave per (work item, kv_head); the group's q heads are processed one
 // after another, each with the per-token online softmax of
@@ -1327,6 +1330,61 @@ uint64_t balanced_work(const std::vector<uint32_t>& positions, uint32_t block_si
     return total + split_segment_pages * segments;
 }
 
+// Chunk length, in pages, of a batch too small to deal out page by page, or 0
+// when it is better dealt out all the same. The times of three plans are
+// weighed in pages of one workgroup alone on its compute unit (k workgroups
+// there share its reads, so a page takes each k times as long): the shortest
+// chunks that make at most k workgroups per compute unit take span * k for each
+// k, and the balanced plan its pages and, for each row, the round trips of one
+// more segment. Rows whose chunks fit one round of workgroups end together;
+// with a few workgroups more than fit, the last round runs nearly alone.
+// Measured on MI355X (8 kv heads of 128, us) against chunks of a quarter of a
+// compute unit's share: 8 rows of 1,000 tokens 11.7 -> 10.6, 4 of 4,000 19.6 ->
+// 16.0, 16 of 1,000 18.6 -> 16.0, 8 of 4,000 29.6 -> 26.0, 24 of U[100, 2500]
+// 29.4 -> 26.1; f32 pages: 8 of 2,000 30.0 -> 24.8, 32 of U[64, 1000] 36.5 ->
+// 26.5; 256-wide heads, 2 kv heads: 32 of U[256, 4096] 47.8 -> 35.6, 32 of 1,000
+// 29.1 -> 19.6.
+uint64_t small_batch_span(const std::vector<uint32_t>& positions, uint32_t block_size,
+                          uint32_t kv_heads, uint64_t cus, const decode_form& form, uint64_t total,
+                          uint64_t longest)
+{
+    const uint64_t rows = positions.size();
+    // a record folded costs about an eighth of a 256-wide page (500 pages of such
+    // heads in chunks of 4, 8 and 16: 17.8, 15.9 and 18.2 us)
+    const uint64_t shortest = std::max<uint64_t>(
+        { form.min_pages, (longest + form.max_chunks - 1) / form.max_chunks,
+          (uint64_t)std::sqrt((double)longest / 8) });
+    uint64_t best_span = 0, best = UINT64_MAX;
+    uint64_t slots = 1;
+    for (uint64_t k = 1; k <= form.per_cu; ++k) {
+        slots = std::max<uint64_t>(1, cus * k / kv_heads);
+        if (rows > slots)
+            continue;
+        // the shortest span of at most `slots` chunks (longest makes one per row)
+        uint64_t lo = std::min(shortest, longest), hi = longest;
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) / 2;
+            uint64_t chunks = 0;
+            for (const uint32_t p : positions)
+                chunks += (p / block_size + mid) / mid;
+            if (chunks <= slots)
+                hi = mid;
+            else
+                lo = mid + 1;
+        }
+        if (hi * k < best || (form.few_waves && hi * k == best)) {
+            best = hi * k;
+            best_span = hi;
+        }
+    }
+    // pages of work the balanced plan gives a compute unit
+    const uint64_t work = form.per_cu * (total + split_row_pages / form.per_cu * rows);
+    const uint64_t dealt = (work + slots - 1) / slots;
+    if (total >= slots * form.min_pages && rows <= slots && 100 * dealt < 97 * best)
+        return 0;
+    return best_span;
+}
+
 uint64_t forced_pages(const char* name, bool& set)
 {
     const char* v = std::getenv(name);
@@ -1342,8 +1400,15 @@ uint32_t decode_fast_waves(uint32_t group, int dtype, uint32_t units, int cu_cou
     return fast_waves(group, dtype, units, cu_count, mean_pages, split_pages);
 }
 
+decode_form decode_form_of(int dtype, uint32_t head_dim)
+{
+    if (dtype == CKV_F32)
+        return form_f32;
+    return head_dim == 256 ? form_wide : form_narrow;
+}
+
 decode_plan_shape shape_decode_plan(const std::vector<uint32_t>& positions, uint32_t block_size,
-                                    uint32_t kv_heads, int cu_count)
+                                    uint32_t kv_heads, int cu_count, const decode_form& form)
 {
     const uint32_t rows = (uint32_t)positions.size();
     decode_plan_shape shape { 0, rows, 0, 0, rows, 0, 0, false };
@@ -1360,32 +1425,43 @@ decode_plan_shape shape_decode_plan(const std::vector<uint32_t>& positions, uint
         const uint64_t cus = (uint64_t)std::max(cu_count, 1);
         const uint64_t share = total * kv_heads / cus;
         // Rows stay whole when they give every compute unit one or two (row,
-        // kv head) units and the longest is within split_uncut_slack of the
-        // share: a cut costs its merge and second segment, about 12 us, and
-        // the cut plan's pages run about 12 % slower than a whole row's. With
-        // more units per compute unit the fixed chunks balance better (the
-        // config-5 churn's batches of hundreds of rows: 1.5 % faster cut).
+        // kv head) units and the longest is within the form's slack of the
+        // share: a cut costs its merge and second segment, and the cut plan's
+        // pages run about 12 % slower than a whole row's. With more units per
+        // compute unit the fixed chunks balance better (the config-5 churn's
+        // batches of hundreds of rows: 1.5 % faster cut).
         const uint64_t units = (uint64_t)rows * kv_heads;
-        const bool fill = units >= cus && units <= 2 * cus;
-        if (2 * longest > share
-            && (!fill || longest > share + share / 8 + split_uncut_slack)) {
+        const bool fill = !form.few_waves && units >= cus && units <= 2 * cus;
+        const uint64_t slack = std::min(share / 8 + form.uncut_slack, 5 * share / 8);
+        // with more than two units per compute unit, whole rows start longest
+        // first and even out while none is over 4/5 of the share (96 and 80
+        // rows of U[100, 3000] tokens whole 99.9 and 86.1 us, in chunks 105.1
+        // and 89.3)
+        const bool even = units > 2 * cus && 5 * longest <= 4 * share;
+        if (2 * longest > share && !even && (!fill || longest > share + slack)) {
             // as many workgroups as the GPU holds at once, but no more than a
             // row each where rows are short (pieces of at least
-            // split_min_pages), nor more than split_max_chunks to a row
-            const uint64_t slots = std::max<uint64_t>(1, cus * split_wgs_per_cu / kv_heads);
-            const uint64_t piece = std::max(split_min_pages,
-                                            (longest + split_max_chunks - 1) / split_max_chunks);
+            // split_min_pages), nor more than max_chunks to a row
+            const uint64_t slots = std::max<uint64_t>(1, cus * form.per_cu / kv_heads);
+            const uint64_t piece = std::max<uint64_t>(
+                form.min_pages, (longest + form.max_chunks - 1) / form.max_chunks);
             deal = std::max<uint64_t>(1, std::min(slots, std::max<uint64_t>(rows, total / piece)));
-            // More rows than workgroups (the balanced plan would run several
-            // whole rows one after another in a workgroup, each paying its
-            // round trips) or too little work per workgroup to pay for a
-            // second segment: fixed chunks instead, a quarter of a compute
-            // unit's share, dispatched longest first.
-            if (rows > deal || total < deal * split_balance_min_pages) {
+            if (rows > deal) {
+                // More rows than workgroups (the balanced plan would run several
+                // whole rows one after another in a workgroup, each paying its
+                // round trips): fixed chunks instead, a quarter of a compute
+                // unit's share, dispatched longest first.
                 deal = 0;
-                span = std::max({ split_min_pages, (share + split_per_share - 1) / split_per_share,
-                                  (longest + split_max_chunks - 1) / split_max_chunks });
+                span = std::max({ (uint64_t)form.min_pages,
+                                  (share + split_per_share - 1) / split_per_share,
+                                  (longest + form.max_chunks - 1) / form.max_chunks });
                 fixed_set = true;
+            } else if (form.per_cu == 1 || total < deal * split_balance_min_pages) {
+                span = small_batch_span(positions, block_size, kv_heads, cus, form, total, longest);
+                if (span) {
+                    deal = 0;
+                    fixed_set = true;
+                }
             }
         }
     }

@@ -31,10 +31,11 @@ uint32_t pages_of(uint32_t position)
 
 // Builds the plan of `positions` (rows' table offsets packed in row order)
 // and checks every structural property; returns it for further checks.
-plan_view plan_and_check(const std::vector<uint32_t>& positions, uint32_t kv_heads, int cus)
+plan_view plan_and_check(const std::vector<uint32_t>& positions, uint32_t kv_heads, int cus,
+                           const ckv::decode_form& form = ckv::decode_form_of(CKV_BF16, 128))
 {
     plan_view v;
-    v.shape = ckv::shape_decode_plan(positions, bs, kv_heads, cus);
+    v.shape = ckv::shape_decode_plan(positions, bs, kv_heads, cus, form);
     std::vector<uint32_t> offsets(positions.size());
     uint32_t at = 0;
     for (size_t r = 0; r < positions.size(); ++r) {
@@ -263,6 +264,36 @@ TEST("forced balance: several rows and pieces to a workgroup (CKV_DECODE_BALANCE
     for (const char* t : { "1", "2", "7" }) {
         const env_guard e("CKV_DECODE_BALANCE", t);
         plan_and_check(p, 8, 256);
+    }
+}
+
+TEST("small batches: chunks that fit one round of workgroups")
+{
+    // equal rows that divide the GPU: 8 of 63 pages in 4 chunks, 4 of 250 in 8,
+    // one workgroup per compute unit
+    auto v = plan_and_check(std::vector<uint32_t>(8, 999), 8, 256);
+    CHECK(!v.shape.balanced && v.shape.n_wgs == 32 && v.shape.split_pages == 16);
+    v = plan_and_check(std::vector<uint32_t>(4, 3999), 8, 256);
+    CHECK(!v.shape.balanced && v.shape.n_wgs == 32 && v.shape.split_pages == 32);
+    // f32: two workgroups of four waves per compute unit
+    v = plan_and_check(std::vector<uint32_t>(8, 1999), 8, 256, ckv::decode_form_of(CKV_F32, 128));
+    CHECK(!v.shape.balanced && v.shape.n_wgs == 64 && v.shape.split_pages == 16);
+    // 256-wide heads: one workgroup per compute unit, 128 per kv head
+    v = plan_and_check(std::vector<uint32_t>(32, 999), 2, 256, ckv::decode_form_of(CKV_BF16, 256));
+    CHECK(!v.shape.balanced && v.shape.n_wgs == 128 && v.shape.split_pages == 16);
+    std::mt19937_64 g(11);
+    for (int t = 0; t < 1500; ++t) {
+        std::vector<uint32_t> p(1 + g() % 100);
+        for (auto& x : p)
+            x = (uint32_t)(g() % ((g() % 3) ? 1200 : 30000));
+        const uint32_t heads = 1 + (uint32_t)(g() % 16);
+        const int cus = 1 + (int)(g() % 320);
+        const auto form = ckv::decode_form_of(g() % 2 ? CKV_F32 : CKV_F16, g() % 2 ? 128 : 256);
+        const auto w = plan_and_check(p, heads, cus, form);
+        // cut into chunks, no more than fit at once, unless there are more rows than that
+        const size_t slots = std::max<size_t>(1, (size_t)cus * form.per_cu / heads);
+        if (w.shape.n_cut && p.size() <= slots)
+            CHECK(w.shape.n_wgs <= slots);
     }
 }
 
