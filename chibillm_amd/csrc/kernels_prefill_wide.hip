@@ -24,6 +24,15 @@
 // sooner than V: K and V have four LDS stages each (131 KB, one workgroup per
 // compute unit), iteration kb loads K(kb + 3) and V(kb + 2), and its barrier
 // publishes K(kb + 2) and V(kb).
+//
+// Four sequences of 300 to 512 rows behind 700 tokens (2 kv heads, 8 q heads,
+// gated) take 50 us for 12.1 GFLOP, where the same rows through the decode
+// kernel took 440: 102 workgroups, their keys in two ranges, so the longest runs
+// 23 blocks one after another. A block takes 3,500 cycles of a wave: 1,000 to
+// issue its loads (about 32 bytes a cycle and compute unit pass to LDS), 890 for
+// the scores and probabilities, 720 for P.V, 700 for maxima, waits and rescales.
+// Issuing the loads in twos between those phases took 64.1 to 64.7 us in all
+// instead of 62.3; reading both halves of V before the scores 64.7.
 #include "ckv_internal.h"
 #include "prefill_records.h"
 #include "prefill_tile.h"
@@ -42,9 +51,13 @@ constexpr uint32_t n_stages = 4;
 constexpr uint32_t k_steps = dim / 16; // products of a block's S^T
 constexpr uint32_t tiles_o = dim / 32; // accumulators of O^T
 
-// K stage: region ks (1 KiB) holds at 16-byte slot 32g + n features 16ks + 8g
-// .. +7 of LDS row n (physical key key_row(n)), the A operand of step ks.
-constexpr uint32_t k_stage_bytes = k_steps * 1024;
+// K stage: the block's 32 key rows of 512 bytes in order, the 16-byte chunks of
+// row k in the order chunk ^ (k % 16): a DMA instruction moves two whole rows
+// (eight full cache lines), and the 16 lanes that read a chunk of 16 rows
+// together find it at 16 different bank offsets (staged in operand order, 32 bytes
+// of each of 32 rows per instruction, the launch below took 62.9 us instead of
+// 62.3).
+constexpr uint32_t k_stage_bytes = block_keys * dim * 2;
 // V stage: two halves of 128 features, each as kernels_prefill.hip stages a
 // 128-wide head: 8 groups of 4 key rows, 64 bytes after each group.
 constexpr uint32_t vg_bytes = 1024 + 64;
@@ -143,9 +156,9 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
     for (uint32_t ks = 0; ks < k_steps; ++ks)
         qr[ks] = *reinterpret_cast<const u32x4_t*>(q + qoff + ks * 16 + g * 8);
 
-    // Staging: the wave moves K regions wave, wave + 4, .. (features 16 * region
-    // ..: 128 bytes apart) and V groups wave, wave + 4 of each half (the block's
-    // first and second page), one DMA each.
+    // Staging: the wave moves K row pairs 2 wave, 2 wave + 8 of each page of the
+    // block and V groups wave, wave + 4 of each half (the block's first and
+    // second page), one DMA each.
     const uint64_t page_bytes = (uint64_t)page_tokens * F * 2;
     const uint64_t base_elems = layer * p.layer_elems + (uint64_t)kvh * dim;
     const uint8_t* kbytes = uniform_ptr(reinterpret_cast<const uint8_t*>(
@@ -153,10 +166,12 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
     const uint8_t* vbytes = uniform_ptr(reinterpret_cast<const uint8_t*>(
         static_cast<const uint16_t*>(p.values) + base_elems));
     const uint8_t* zbytes = reinterpret_cast<const uint8_t*>(zero_row);
-    const uint32_t k_key = key_row(n); // this lane's key in a block, and its bytes into the page
-    const bool k_hi = k_key >= page_tokens;
-    const uint32_t k_feat = 16 * wave + 8 * g;
-    const uint32_t k_off = ((k_key & 15) * F + k_feat) * 2;
+    uint32_t k_row[2], k_off[2]; // this lane's key of a page and its source bytes there
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+        k_row[i] = 2 * wave + 8 * i + g;
+        k_off[i] = k_row[i] * F * 2 + (n ^ k_row[i]) * 16;
+    }
     const uint32_t v_key = 4 * (lane >> 4) + wave; // in either page
     const uint32_t v_off = (v_key * F + (lane & 15) * 8) * 2;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -171,21 +186,22 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
     auto page_of = [&](uint32_t entry) { // a scalar load; past the tile's end, its last page
         return *(c32*)(table_s + 4 * (uint64_t)min(entry, last_entry));
     };
+    auto page_at = [&](uint32_t page) { // a page's bytes from the layer's base
+        return FAR ? page * page_bytes : (uint64_t)(page * (uint32_t)page_bytes);
+    };
     auto load_k = [&](uint32_t kb, uint32_t pg0, uint32_t pg1) {
-        const uint32_t st = lds_base + k_stage(kb) + wave * 1024;
-        const bool whole = kb * block_keys + block_keys - 1 <= pos_last;
-        if (!FAR && whole) {
-            const uint32_t off = (k_hi ? pg1 : pg0) * (uint32_t)page_bytes + k_off;
+        const uint32_t key0 = kb * block_keys;
+        const bool whole = key0 + block_keys - 1 <= pos_last;
 #pragma unroll
-            for (uint32_t r = 0; r < regions; ++r)
-                dma16_s(kbytes + 128 * r, off, st + r * waves * 1024);
-        } else {
-            const uint8_t* src = kbytes + (k_hi ? pg1 : pg0) * page_bytes + k_off;
-            if (kb * block_keys + k_key > pos_last)
-                src = zbytes + k_feat * 2;
-#pragma unroll
-            for (uint32_t r = 0; r < regions; ++r)
-                dma16(src + 128 * r, st + r * waves * 1024);
+        for (uint32_t r = 0; r < regions; ++r) { // the block's page r / 2, rows 8 * (r % 2) ..
+            const uint32_t st = lds_base + k_stage(kb) + (wave + 4 * r) * 1024;
+            const uint8_t* pk = kbytes + page_at(r / 2 ? pg1 : pg0);
+            if (whole) {
+                dma16_s(pk, k_off[r % 2], st);
+            } else {
+                const bool live = key0 + page_tokens * (r / 2) + k_row[r % 2] <= pos_last;
+                dma16(live ? pk + k_off[r % 2] : zbytes + n * 16, st);
+            }
         }
     };
     auto load_v = [&](uint32_t kb, uint32_t pg0, uint32_t pg1) {
@@ -195,7 +211,7 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
         for (uint32_t r = 0; r < regions; ++r) { // half r / 2, the block's page r % 2
             const uint32_t st = lds_base + v_stage(kb) + (r / 2) * v_half_bytes
                 + (wave + 4 * (r % 2)) * vg_bytes;
-            const uint8_t* pv = vbytes + (r % 2 ? pg1 : pg0) * page_bytes + 256 * (r / 2);
+            const uint8_t* pv = vbytes + page_at(r % 2 ? pg1 : pg0) + 256 * (r / 2);
             if (whole) {
                 dma16_s(pv, v_off, st);
             } else {
@@ -216,24 +232,29 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
     float mx = 0.0f;
     uint4 ka[k_steps];
 
+    // A operand of step ks: chunk 2ks + g of key row key_row(n)
+    const uint32_t kr_row = key_row(n) * (dim * 2), kr_swap = ((key_row(n) & 15) ^ g) * 16;
     auto read_k = [&](uint32_t kb) {
-        const uint8_t* kl = lds + k_stage(kb) + lane * 16;
+        const uint32_t base = lds_base + k_stage(kb) + kr_row;
 #pragma unroll
-        for (uint32_t ks = 0; ks < k_steps; ++ks)
-            ka[ks] = *reinterpret_cast<const uint4*>(kl + ks * 1024);
+        for (uint32_t ks = 0; ks < k_steps; ++ks) {
+            const uint32_t at = base + (kr_swap ^ (32 * (ks % 8))); // chunk bit 4 is not swapped
+            ka[ks] = __builtin_bit_cast(uint4, *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)(at + 256 * (ks / 8)));
+        }
     };
     const uint32_t vr_off = ((lane & 15) >> 2) * vg_bytes + (lane >> 5) * 512
         + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
-    // A operand of O^T's accumulator mt: features 32mt + n, keys 16h + 8g + 0..7
-    auto read_v = [&](uint32_t kb, uint4 (&va)[tiles_o][2]) {
-        uint32_t vaddr = lds_base + v_stage(kb) + vr_off;
+    // A operands of O^T's accumulators 4 * half + mt (features 32mt + n of that
+    // half of the head), keys 16h + 8g + 0..7
+    auto read_v = [&](uint32_t kb, uint32_t half, uint4 (&va)[4][2]) {
+        uint32_t vaddr = lds_base + v_stage(kb) + half * v_half_bytes + vr_off;
         asm volatile("" : "+v"(vaddr));
         auto* vb = (__attribute__((address_space(3))) uint8_t*)(uintptr_t)vaddr;
 #pragma unroll
-        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+        for (uint32_t mt = 0; mt < 4; ++mt)
 #pragma unroll
             for (uint32_t h = 0; h < 2; ++h) {
-                auto* at = vb + (mt / 4) * v_half_bytes + 4 * h * vg_bytes + 64 * (mt % 4);
+                auto* at = vb + 4 * h * vg_bytes + 64 * mt;
                 const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                     (__attribute__((address_space(3))) i16x4_t*)at);
                 const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -273,17 +294,18 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
 #pragma unroll
         for (uint32_t ks = 0; ks < k_steps; ++ks)
             s = mfma<F16>(ka[ks], __builtin_bit_cast(uint4, qr[ks]), s);
+        asm volatile("" : "+v"(s)); // the vector ALU reads it next
         return s;
     };
-    auto pv = [&](const uint4 (&va)[tiles_o][2], const uint4 (&hi)[2], const uint4 (&lo)[2]) {
+    auto pv = [&](uint32_t half, const uint4 (&va)[4][2], const uint4 (&hi)[2], const uint4 (&lo)[2]) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
-            for (uint32_t mt = 0; mt < tiles_o; ++mt)
-                o[mt] = mfma<F16>(va[mt][h], hi[h], o[mt]);
+            for (uint32_t mt = 0; mt < 4; ++mt)
+                o[4 * half + mt] = mfma<F16>(va[mt][h], hi[h], o[4 * half + mt]);
 #pragma unroll
-            for (uint32_t mt = 0; mt < tiles_o; ++mt)
-                o[mt] = mfma<F16>(va[mt][h], lo[h], o[mt]);
+            for (uint32_t mt = 0; mt < 4; ++mt)
+                o[4 * half + mt] = mfma<F16>(va[mt][h], lo[h], o[4 * half + mt]);
         }
     };
     // causal mask and maxima of block kb's scores, which become sp
@@ -291,6 +313,7 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
         sp = s;
         const uint32_t key0 = kb * block_keys;
         if (key0 + block_keys - 1 > pos_lo) {
+            asm volatile(""); // a branch: most blocks end before the diagonal
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const uint32_t kpos = key0 + 16 * (r >> 3) + 8 * g + (r & 7);
@@ -310,8 +333,10 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
         m = m_new;
         m_limit = m_new + rescale_raw;
 #pragma unroll
-        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+        for (uint32_t mt = 0; mt < tiles_o; ++mt) {
             o[mt] *= alpha;
+            asm volatile("" : "+a"(o[mt])); // one accumulator at a time, see pin
+        }
     };
 
     // Before the loop: blocks b .. b + 3 of K and b .. b + 2 of V, those that
@@ -374,21 +399,20 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
     };
     for (uint32_t kb = kb_begin + 1; kb < kb_end; ++kb) {
         pin();
-        uint32_t newest = kb + 2 < kb_end ? regions : 0;
-        if (kb + 3 < kb_end) {
+        const bool more_k = kb + 3 < kb_end, more_v = kb + 2 < kb_end;
+        const uint32_t newest = (more_v ? 2 * regions : 0) + (more_k ? regions : 0);
+        if (more_k)
             load_k(kb + 3, pk0, pk1);
-            newest += regions;
-        }
-        if (kb + 2 < kb_end) {
+        if (more_v)
             load_v(kb + 2, pw0, pw1);
-            newest += regions;
-        }
-        uint4 va[tiles_o][2], hi[2], lo[2];
-        read_v(kb - 1, va);
-        const f32x16_t s = qk();   // matrix: block kb
-        probabilities(hi, lo);     // vector: block kb - 1
+        uint4 va[4][2], vb[4][2], hi[2], lo[2];
+        read_v(kb - 1, 0, va);
+        const f32x16_t s = qk(); // matrix: block kb
+        probabilities(hi, lo);   // vector: block kb - 1
+        read_v(kb - 1, 1, vb);
+        pv(0, va, hi, lo); // matrix: block kb - 1
         read_k(min(kb + 1, kb_end - 1)); // past the range's end: any staged block
-        pv(va, hi, lo);            // matrix: block kb - 1
+        pv(1, vb, hi, lo);
         pw0 = pk0;
         pw1 = pk1;
         pk0 = page_of(2 * (kb + 4));
@@ -400,10 +424,13 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
             rescale();
     }
     {
-        uint4 va[tiles_o][2], hi[2], lo[2];
-        read_v(kb_end - 1, va);
+        uint4 va[4][2], hi[2], lo[2];
         probabilities(hi, lo);
-        pv(va, hi, lo);
+#pragma unroll
+        for (uint32_t half = 0; half < 2; ++half) {
+            read_v(kb_end - 1, half, va);
+            pv(half, va, hi, lo);
+        }
     }
 
     float lt = l + __shfl_xor(l, 32); // the query's denominator (both lane halves)
