@@ -93,6 +93,85 @@ __device__ __forceinline__ void wait_all_but(uint32_t loads)
         __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
+// One query vector against keys 0 .. pos by vector arithmetic: what its wave falls
+// back to when the tile gave it a value that is not finite. A product with
+// P^T multiplies every key of a block for all its queries, so an infinity or NaN
+// in a V row also meets the zeros of the queries that do not attend it (and of a
+// low term), and 0 * inf is NaN; the decode kernels give such a row only to the
+// queries that attend it, and so does this. Sixteen lanes hold a row, four rows
+// a step; finite results never come here.
+template <bool F16>
+__device__ __forceinline__ void attend_alone(const uint16_t* __restrict__ keys,
+                                             const uint16_t* __restrict__ values,
+                                             const uint32_t* __restrict__ table, uint32_t F,
+                                             uint32_t pos, const uint16_t* q, float c,
+                                             const uint16_t* gate, uint16_t* out, uint32_t lane)
+{
+    constexpr uint32_t each = dim / 16;
+    const uint32_t f = (lane & 15) * each, sub = lane >> 4;
+    auto features = [](const uint16_t* at, float (&x)[each]) {
+        const u32x4_t w[2] = { reinterpret_cast<const u32x4_t*>(at)[0],
+                               reinterpret_cast<const u32x4_t*>(at)[1] };
+#pragma unroll
+        for (uint32_t i = 0; i < each; ++i)
+            x[i] = word_value<F16>(w[i / 8][i / 2 % 4], i % 2);
+    };
+    auto weight = [&](float ms, float to) { // 0 for a share that attended nothing
+        return ms == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((ms - to) * c);
+    };
+    float qf[each], acc[each] = {}, m = -__builtin_inff(), l = 0.0f;
+    features(q + f, qf);
+    for (uint32_t key0 = 0; key0 <= pos; key0 += page_tokens) {
+        const uint64_t page = (uint64_t)table[key0 / page_tokens] * page_tokens;
+#pragma unroll 1
+        for (uint32_t i = 0; i < page_tokens / 4; ++i) {
+            const uint32_t key = key0 + 4 * i + sub;
+            const uint64_t at = (page + min(key, pos) % page_tokens) * F + f;
+            float x[each], s = 0.0f;
+            features(keys + at, x);
+#pragma unroll
+            for (uint32_t j = 0; j < each; ++j)
+                s = __builtin_fmaf(qf[j], x[j], s);
+#pragma unroll
+            for (uint32_t d = 1; d < 16; d *= 2)
+                s += __shfl_xor(s, d);
+            features(values + at, x);
+            if (key <= pos) {
+                const float m_new = fmaxf(m, s), keep = weight(m, m_new), w = weight(s, m_new);
+                m = m_new;
+                l = l * keep + w;
+#pragma unroll
+                for (uint32_t j = 0; j < each; ++j)
+                    acc[j] = acc[j] * keep + w * x[j];
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t d = 16; d < 64; d *= 2) {
+        const float m_other = __shfl_xor(m, d), l_other = __shfl_xor(l, d);
+        const float m_new = fmaxf(m, m_other);
+        const float keep = weight(m, m_new), w = weight(m_other, m_new);
+        m = m_new;
+        l = l * keep + l_other * w;
+#pragma unroll
+        for (uint32_t j = 0; j < each; ++j) {
+            const float other = __shfl_xor(acc[j], d);
+            acc[j] = (keep > 0.0f ? acc[j] * keep : 0.0f) + (w > 0.0f ? other * w : 0.0f);
+        }
+    }
+    if (sub)
+        return;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (uint32_t j = 0; j < each; j += 2) {
+        float x[2] = { acc[j] * inv, acc[j + 1] * inv };
+        if (gate)
+            for (int e = 0; e < 2; ++e)
+                x[e] *= sigmoid(half_value<F16>(gate[f + j + e]));
+        *reinterpret_cast<uint32_t*>(out + f + j) = pack2<F16>(x[0], x[1]);
+    }
+}
+
 // FAR: a layer spans more than 4 GiB, so page offsets take 64 bits.
 template <int G, bool F16, bool FAR>
 __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
@@ -503,27 +582,43 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
         }
     }
 
-    if (!valid)
-        return;
     const float inv = 1.0f / lt;
-    uint16_t* dst = out + qoff;
+    // 0 unless some result of the query is infinite or NaN (either lane half)
+    float odd = inv * 0.0f;
 #pragma unroll
     for (uint32_t mt = 0; mt < tiles_o; ++mt)
 #pragma unroll
-        for (uint32_t quad = 0; quad < 4; ++quad) {
-            const uint32_t f = 32 * mt + 8 * quad + 4 * g;
-            float x[4] = { o[mt][4 * quad] * inv, o[mt][4 * quad + 1] * inv,
-                           o[mt][4 * quad + 2] * inv, o[mt][4 * quad + 3] * inv };
-            if (gate) { // sigmoid_mul (src/qwen/qwen_layer.cc:204) in the epilogue
-                const uint2 gv = *reinterpret_cast<const uint2*>(gate + qoff + f);
-                const uint32_t w[2] = { gv.x, gv.y };
+        for (int r = 0; r < 16; ++r)
+            odd = __builtin_fmaf(o[mt][r], 0.0f, odd);
+    const uint64_t odd_lanes = __ballot(valid && odd != 0.0f);
+    const uint32_t alone = (uint32_t)odd_lanes | (uint32_t)(odd_lanes >> 32);
+    uint16_t* dst = out + qoff;
+    if (valid && !(alone >> n & 1)) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    x[e] *= sigmoid(half_value<F16>((uint16_t)(w[e / 2] >> (16 * (e % 2)))));
+        for (uint32_t mt = 0; mt < tiles_o; ++mt)
+#pragma unroll
+            for (uint32_t quad = 0; quad < 4; ++quad) {
+                const uint32_t f = 32 * mt + 8 * quad + 4 * g;
+                float x[4] = { o[mt][4 * quad] * inv, o[mt][4 * quad + 1] * inv,
+                               o[mt][4 * quad + 2] * inv, o[mt][4 * quad + 3] * inv };
+                if (gate) { // sigmoid_mul (src/qwen/qwen_layer.cc:204) in the epilogue
+                    const uint2 gv = *reinterpret_cast<const uint2*>(gate + qoff + f);
+                    const uint32_t w[2] = { gv.x, gv.y };
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        x[e] *= sigmoid(half_value<F16>((uint16_t)(w[e / 2] >> (16 * (e % 2)))));
+                }
+                *reinterpret_cast<uint2*>(dst + f) =
+                    make_uint2(pack2<F16>(x[0], x[1]), pack2<F16>(x[2], x[3]));
             }
-            *reinterpret_cast<uint2*>(dst + f) =
-                make_uint2(pack2<F16>(x[0], x[1]), pack2<F16>(x[2], x[3]));
-        }
+    }
+    for (uint32_t left = alone; left; left &= left - 1) {
+        const uint32_t r = rb * 32 + __builtin_ctz(left);
+        const size_t at = (size_t)(row0 + r) * q_stride + (size_t)head * dim;
+        attend_alone<F16>(static_cast<const uint16_t*>(p.keys) + base_elems,
+                          static_cast<const uint16_t*>(p.values) + base_elems, table, F, pos0 + r,
+                          q + at, c, gate ? gate + at : nullptr, out + at, lane);
+    }
 }
 
 template <int G>

@@ -196,3 +196,53 @@ def test_wide_prefill_matches_oracle_and_general_path(ctx, code, group, gated, s
         assert_close(got, expected, what="prefill")
         off, off_general = (np.linalg.norm(x - expected) for x in (got, general))
         assert off <= 1.1 * off_general, (off, off_general)
+
+
+@pytest.mark.parametrize("code,group,gated,split", [
+    (orc.BF16, 4, True, "1"), (orc.F16, 2, False, "4"), (orc.BF16, 8, False, "2"), (orc.F16, 1, True, "1")])
+def test_wide_prefill_keeps_values_that_are_not_finite_with_their_rows(ctx, code, group, gated, split,
+                                                                       monkeypatch):
+    """Infinities and a NaN among the keys and values reach exactly the rows
+    that attend them, as in the general path: a query of the same tile that stands
+    before such a token has none of it, and an infinite value stays an infinity."""
+    print(f"wide prefill, not finite: dtype {code} group {group} gated {gated} split {split}", flush=True)
+    monkeypatch.setenv("CKV_PREFILL_SPLIT", split)
+    monkeypatch.setenv("CKV_PREFILL_SPLIT_MIN", "1")
+    rng = orc.Mt64(1500 + 10 * group + code)
+    H, prefix, rows = 2, 21, 150
+    span, Hq, F = prefix + rows, H * group, H * D
+    pages = -(-span // 16)
+    geom, table = (1, pages + 1, 16, H, D), rng.permutation(pages + 1)[:pages]
+    k, v = (rng.normal(span * F, code).reshape(span, F).copy() for _ in range(2))
+    q = rng.normal(rows * Hq * D, code).reshape(rows, -1)
+    gate = rng.normal(rows * Hq * D, code).reshape(rows, -1)
+    inf, nan = (0x7F80, 0x7FC0) if code == orc.BF16 else (0x7C00, 0x7E00)
+    v[40, 3] = v[77, 200] = inf          # kv head 0, two features
+    v[60, D + 9] = v[61, D + 9] = inf | 0x8000  # kv head 1
+    k[130, 5] = inf                      # scores of one sign or the other
+    v[150, D + 30] = nan
+    kc, vc = nan_pages(code, geom[1] * 16 * F), nan_pages(code, geom[1] * 16 * F)
+    orc.store_kv(kc, vc, k, v, [orc.slot(table, p, 16) for p in range(span)], 0, geom[1] * 16)
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(to_dev(vc, code))
+    pool.upload(table, np.zeros(rows, np.uint32), np.full(rows, pages),
+                np.arange(prefix, span).astype(np.uint32))
+    outs = []
+    for shift in (lambda t: t, misaligned):
+        qd = shift(to_dev(q, code))
+        out = shift(torch.full((rows, Hq * D), float("nan"), dtype=qd.dtype, device="cuda"))
+        if gated:
+            pool.attention_gated(0, qd, Hq, 1 / math.sqrt(D), to_dev(gate, code), out)
+        else:
+            pool.attention(0, qd, Hq, 1 / math.sqrt(D), out)
+        ctx.sync()
+        outs.append(orc.to_f32(to_host(out, code), code).reshape(rows, Hq * D))
+    pool.close()
+    got, general = outs
+    assert np.isfinite(general[:40 - prefix]).all() and np.isinf(general).any() and np.isnan(general).any()
+    assert np.array_equal(np.isnan(got), np.isnan(general))
+    assert np.array_equal(np.isinf(got), np.isinf(general))
+    fin = np.isfinite(general)
+    assert_close(got[fin], general[fin], what="finite values")
+    assert np.array_equal(np.sign(got[~fin & ~np.isnan(got)]), np.sign(general[~fin & ~np.isnan(general)]))
