@@ -115,22 +115,24 @@ __global__ __launch_bounds__(block_threads) void rope_kernel(
     }
 }
 
-// 16-bit rows with rotary == head_dim and half a head a multiple of 8: a
-// thread rotates 8 consecutive pairs, reading and writing 16 bytes of each
-// half (two 128-bit loads and stores per tensor instead of sixteen 2-byte
-// accesses). A row's angles are the same for every head, so the workgroup
+// 16-bit rows whose head and rotary widths are multiples of 16: a thread rotates
+// 8 consecutive pairs, reading and writing 16 bytes of each half (two 128-bit
+// loads and stores per tensor instead of sixteen 2-byte accesses), or copies 16
+// elements past the rotary width (16,384 rows of 8 heads of 256, a quarter of
+// each rotated: 41.9 -> 22.8 us against the per-pair kernel, whose 2-byte accesses
+// bound it; 1,624 rows 6.3 -> 5.0). A row's angles are the same for every head, so the workgroup
 // computes the (cosine, sine) of each (row, pair) its threads touch into LDS,
 // one sincosf per entry instead of one per (row, head, pair), while its
 // threads' loads are in flight.
 template <int DT, bool APPEND>
 __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
     const void* in, void* out, uint32_t rows, uint32_t heads, uint32_t head_dim,
-    rope_table freq, const uint32_t* __restrict__ positions, pool_view p,
+    uint32_t rotary, rope_table freq, const uint32_t* __restrict__ positions, pool_view p,
     const uint32_t* __restrict__ slots, uint32_t layer, const void* __restrict__ values)
 {
     using E = element<DT>;
     extern __shared__ float2 angles[]; // (cosine, sine) per (row of the workgroup, pair)
-    const uint32_t half = head_dim / 2, groups = half / 8;
+    const uint32_t half = rotary / 2, groups = head_dim / 16;
     const uint32_t per_row = heads * groups;
     const uint64_t total = (uint64_t)rows * per_row;
     const uint64_t first = (uint64_t)blockIdx.x * block_threads;
@@ -142,15 +144,18 @@ __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
     const uint64_t t = min(first + threadIdx.x, total - 1);
     const uint32_t row = (uint32_t)(t / per_row), rest = (uint32_t)(t % per_row);
     const uint32_t head = rest / groups, p0 = (rest % groups) * 8;
+    const bool rotates = p0 < half;
+    // the item's first element in the head, and its second eight's distance
+    const uint32_t at = rotates ? p0 : 2 * p0, apart = rotates ? half : 8;
     const uint64_t width = (uint64_t)heads * head_dim;
-    const uint64_t src = row * width + head * head_dim + p0;
+    const uint64_t src = row * width + head * head_dim + at;
     const uint4 a = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(in) + src);
-    const uint4 b = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(in) + src + half);
+    const uint4 b = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(in) + src + apart);
     uint4 va = make_uint4(0, 0, 0, 0), vb = va;
     if constexpr (APPEND) {
         const uint16_t* vs = static_cast<const uint16_t*>(values) + src;
         va = *reinterpret_cast<const uint4*>(vs);
-        vb = *reinterpret_cast<const uint4*>(vs + half);
+        vb = *reinterpret_cast<const uint4*>(vs + apart);
     }
     for (uint32_t e = threadIdx.x; e < entries; e += block_threads) {
         const uint32_t r = first_row + e / half, pair = e % half;
@@ -161,7 +166,7 @@ __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
     __syncthreads();
     if (first + threadIdx.x >= total)
         return;
-    const float2* cs = angles + (row - first_row) * half + p0;
+    const float2* cs = angles + (row - first_row) * half + (rotates ? p0 : 0);
     const uint32_t wa[4] = { a.x, a.y, a.z, a.w }, wb[4] = { b.x, b.y, b.z, b.w };
     uint32_t ra[4], rb[4];
 #pragma unroll
@@ -174,6 +179,10 @@ __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
             const float2 c = cs[2 * d + h];
             float r1, r2;
             rope_pair(x1, x2, c.x, c.y, r1, r2);
+            if (!rotates) {
+                r1 = x1;
+                r2 = x2;
+            }
             oa |= static_cast<uint32_t>(E::store(r1)) << (16 * h);
             ob |= static_cast<uint32_t>(E::store(r2)) << (16 * h);
         }
@@ -183,16 +192,16 @@ __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
     uint16_t* dst;
     if constexpr (APPEND) {
         const uint64_t off = layer * p.layer_elems + (uint64_t)slots[row] * p.features
-            + head * head_dim + p0;
+            + head * head_dim + at;
         dst = static_cast<uint16_t*>(p.keys) + off;
         uint16_t* vd = static_cast<uint16_t*>(p.values) + off;
         *reinterpret_cast<uint4*>(vd) = va;
-        *reinterpret_cast<uint4*>(vd + half) = vb;
+        *reinterpret_cast<uint4*>(vd + apart) = vb;
     } else {
         dst = static_cast<uint16_t*>(out) + src;
     }
     *reinterpret_cast<uint4*>(dst) = make_uint4(ra[0], ra[1], ra[2], ra[3]);
-    *reinterpret_cast<uint4*>(dst + half) = make_uint4(rb[0], rb[1], rb[2], rb[3]);
+    *reinterpret_cast<uint4*>(dst + apart) = make_uint4(rb[0], rb[1], rb[2], rb[3]);
 }
 
 bool aligned16(const void* ptr)
@@ -208,7 +217,7 @@ hipError_t launch(hipStream_t s, int dtype, const void* in, void* out, uint32_t 
 {
     if (!rows)
         return hipSuccess;
-    const bool x8 = dtype != CKV_F32 && rotary == head_dim && (head_dim / 2) % 8 == 0
+    const bool x8 = dtype != CKV_F32 && rotary && rotary % 16 == 0 && head_dim % 16 == 0
         && aligned16(in) && (APPEND ? aligned16(values) && aligned16(p.keys) && aligned16(p.values)
                                     : aligned16(out));
     if (x8) {
@@ -218,15 +227,15 @@ hipError_t launch(hipStream_t s, int dtype, const void* in, void* out, uint32_t 
         if (blocks > 0x7FFFFFFFull)
             return hipErrorInvalidValue;
         const dim3 grid((uint32_t)blocks);
-        // the angle table: the rows a workgroup's items fall in, half a head each
+        // the angle table: the rows a workgroup's items fall in, half a rotary width each
         const uint32_t table_rows = std::min<uint32_t>(rows, (block_threads - 1) / per_row + 2);
-        const size_t lds = (size_t)table_rows * (head_dim / 2) * sizeof(float2);
+        const size_t lds = (size_t)table_rows * (rotary / 2) * sizeof(float2);
         if (dtype == CKV_BF16)
             rope_kernel_x8<CKV_BF16, APPEND><<<grid, block_threads, lds, s>>>(
-                in, out, rows, heads, head_dim, freq, positions, p, slots, layer, values);
+                in, out, rows, heads, head_dim, rotary, freq, positions, p, slots, layer, values);
         else
             rope_kernel_x8<CKV_F16, APPEND><<<grid, block_threads, lds, s>>>(
-                in, out, rows, heads, head_dim, freq, positions, p, slots, layer, values);
+                in, out, rows, heads, head_dim, rotary, freq, positions, p, slots, layer, values);
         return hipGetLastError();
     }
     const uint32_t threads = heads * (head_dim / 2);

@@ -113,7 +113,7 @@ def test_rope_validation_codes(ctx):
 def test_rope_append_matches_rope_then_store(ctx, code, rotary):
     """Qwen3-0.6B KV rows (8 heads x 128, theta 1e6) at positions up to 16 K,
     scattered through a permuted table; full width (the 128-bit path for
-    16-bit rows) and a partial rotary width (the per-pair path)."""
+    16-bit rows) and a partial rotary width."""
     print(f"rope_append dtype {code} rotary {rotary}", flush=True)
     rng = orc.Mt64(17 + code)
     H, D, bs, B = 8, 128, 16, 96
@@ -309,3 +309,45 @@ def test_rope_append_decode_validation_codes(ctx):
                                     out, args["rotary_dim"], args["gate"], args["rows"])
         assert e.value.name == name, kwargs
     pool.close()
+
+
+def one_past(t):
+    """A copy one element past a 16-byte boundary."""
+    base = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    view = base[1:1 + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("code", [orc.BF16, orc.F16])
+@pytest.mark.parametrize("heads,dim,rotary", [(1, 16, 16), (3, 32, 16), (2, 256, 64), (5, 128, 96),
+                                              (1, 272, 256), (8, 64, 48), (2, 1024, 16)])
+def test_partial_rotary_in_16_byte_accesses_equals_per_pair(ctx, code, heads, dim, rotary):
+    """Widths that are multiples of 16 move 16 bytes at a time; misaligned rows
+    take the per-pair kernel. The same bits, out of place, in place and appended, with
+    a NaN, infinities and a zero at the head's end among them."""
+    print(f"partial rotary {code} {heads} x {dim} rotary {rotary}", flush=True)
+    rng = orc.Mt64(70 + dim + rotary)
+    rows, B = 37, 4
+    positions = [rng.uniform_int(0, 16383) for _ in range(rows)]
+    x = rng.normal(rows * heads * dim, code).reshape(rows, heads * dim).copy()
+    exponent = 0x7F80 if code == orc.BF16 else 0x7C00
+    x[3, dim - 4:dim] = [exponent, exponent | 1, 0x8000, exponent | 0x8000]
+    v = rng.normal(rows * heads * dim, code).reshape(rows, -1)
+    table = np.arange(1024) % B
+    slots = rng.permutation(B * 16)[:rows]
+    results = []
+    for shift in (lambda t: t, one_past):
+        pool, kd, vd = new_pool(ctx, (1, B, 16, heads, dim), code)
+        pool.upload(table, [0] * rows, [1024] * rows, positions, slots)
+        src = shift(to_dev(x, code))
+        out = shift(torch.zeros_like(src))
+        pool.rope(src, out, heads, 1e6, rotary)
+        pool.rope_append(0, src, shift(to_dev(v, code)), 1e6, rotary)
+        pool.rope(src, src, heads, 1e6, rotary)
+        ctx.sync()
+        results.append([to_host(t, code) for t in (out.clone(), src.clone(), kd, vd)])
+        pool.close()
+    for got, want in zip(*results):
+        assert np.array_equal(got, want)
+    assert np.array_equal(results[0][0], results[0][1])
