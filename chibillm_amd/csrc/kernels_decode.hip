@@ -13,7 +13,7 @@
 // row, two rows per load instruction and half a page per step, which keeps the
 // registers of the 128-wide form; they are read once for the whole group
 // instead of once per q head by one wave (the general path): 32 rows of
-// U[256, 4096] tokens, 2 kv heads, 8 q heads, rotated and gated, 607 -> 57 us. Scores are kept in the log2
+// U[256, 4096] tokens, 2 kv heads, 8 q heads, rotated and gated, 607 -> 37 us. Scores are kept in the log2
 // domain (scale * log2(e)) so every exponential is one v_exp_f32. Rows the
 // batch plan cuts are merged in the same launch with weights 2^(m_c - M), the
 // reduction of paged_attention_reduce_f32
