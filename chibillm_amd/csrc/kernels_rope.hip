@@ -124,7 +124,8 @@ __global__ __launch_bounds__(block_threads) void rope_kernel(
 // computes the (cosine, sine) of each (row, pair) its threads touch into LDS,
 // one sincosf per entry instead of one per (row, head, pair), while its
 // threads' loads are in flight.
-template <int DT, bool APPEND>
+// WHOLE: rotary == head_dim, so no thread copies.
+template <int DT, bool APPEND, bool WHOLE>
 __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
     const void* in, void* out, uint32_t rows, uint32_t heads, uint32_t head_dim,
     uint32_t rotary, rope_table freq, const uint32_t* __restrict__ positions, pool_view p,
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
 {
     using E = element<DT>;
     extern __shared__ float2 angles[]; // (cosine, sine) per (row of the workgroup, pair)
-    const uint32_t half = rotary / 2, groups = head_dim / 16;
+    const uint32_t half = (WHOLE ? head_dim : rotary) / 2, groups = head_dim / 16;
     const uint32_t per_row = heads * groups;
     const uint64_t total = (uint64_t)rows * per_row;
     const uint64_t first = (uint64_t)blockIdx.x * block_threads;
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(block_threads) void rope_kernel_x8(
     const uint64_t t = min(first + threadIdx.x, total - 1);
     const uint32_t row = (uint32_t)(t / per_row), rest = (uint32_t)(t % per_row);
     const uint32_t head = rest / groups, p0 = (rest % groups) * 8;
-    const bool rotates = p0 < half;
+    const bool rotates = WHOLE || p0 < half;
     // the item's first element in the head, and its second eight's distance
     const uint32_t at = rotates ? p0 : 2 * p0, apart = rotates ? half : 8;
     const uint64_t width = (uint64_t)heads * head_dim;
@@ -230,12 +231,12 @@ hipError_t launch(hipStream_t s, int dtype, const void* in, void* out, uint32_t 
         // the angle table: the rows a workgroup's items fall in, half a rotary width each
         const uint32_t table_rows = std::min<uint32_t>(rows, (block_threads - 1) / per_row + 2);
         const size_t lds = (size_t)table_rows * (rotary / 2) * sizeof(float2);
-        if (dtype == CKV_BF16)
-            rope_kernel_x8<CKV_BF16, APPEND><<<grid, block_threads, lds, s>>>(
-                in, out, rows, heads, head_dim, rotary, freq, positions, p, slots, layer, values);
-        else
-            rope_kernel_x8<CKV_F16, APPEND><<<grid, block_threads, lds, s>>>(
-                in, out, rows, heads, head_dim, rotary, freq, positions, p, slots, layer, values);
+        const bool whole = rotary == head_dim;
+        auto* kernel = dtype == CKV_BF16
+            ? (whole ? rope_kernel_x8<CKV_BF16, APPEND, true> : rope_kernel_x8<CKV_BF16, APPEND, false>)
+            : (whole ? rope_kernel_x8<CKV_F16, APPEND, true> : rope_kernel_x8<CKV_F16, APPEND, false>);
+        kernel<<<grid, block_threads, lds, s>>>(in, out, rows, heads, head_dim, rotary, freq,
+                                                positions, p, slots, layer, values);
         return hipGetLastError();
     }
     const uint32_t threads = heads * (head_dim / 2);
