@@ -55,3 +55,42 @@ def test_merges_at_every_remainder(ctx, code, dim, group, monkeypatch):
             else:
                 assert_close(orc.to_f32(got, code), expected, what=f"{waves} waves, split {split}")
     pool.close()
+
+
+@pytest.mark.parametrize("code,dim,group", [(orc.BF16, 128, 2), (orc.F32, 128, 1), (orc.F16, 256, 4)])
+def test_merges_keep_infinities(ctx, code, dim, group, monkeypatch):
+    """An infinite value stays an infinity, whichever wave's or slice's state
+    holds it: every third token but a row's last has one, at a feature of its own
+    (positive at even ones), so each state and record has some."""
+    H, Hq, rows = 2, 2 * group, len(LENGTHS)
+    rng = orc.Mt64(340 + dim + code)
+    pages = [-(-n // 16) for n in LENGTHS]
+    blocks = sum(pages)
+    flat, offsets = rng.permutation(blocks), np.cumsum([0] + pages[:-1])
+    tables = np.split(flat, offsets[1:])
+    geom = (1, blocks, 16, H, dim)
+    kc = rng.normal(blocks * 16 * H * dim, code)
+    v = rng.normal(blocks * 16 * H * dim, orc.F32).reshape(-1, H, dim)
+    infinite = np.zeros((rows, dim))
+    for r, n in enumerate(LENGTHS):
+        for t in range(0, n - 1, 3):
+            f = t % dim
+            infinite[r, f] = -np.inf if f % 2 else np.inf
+            v[orc.slot(tables[r], t, 16), :, f] = infinite[r, f]
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(torch.from_numpy(v.reshape(-1)).to(vd.dtype))
+    qd = to_dev(rng.normal(rows * Hq * dim, code).reshape(rows, -1), code)
+    where = np.broadcast_to(infinite[:, None], (rows, Hq, dim))
+    for waves in (1, 2, 3, 5, 6, 7, 8, 10):
+        for split in (1, 2, 3, 4, 7, 0):
+            monkeypatch.setenv("CKV_DECODE_WAVES", str(waves))
+            monkeypatch.setenv("CKV_DECODE_SPLIT", str(split))
+            pool.upload(flat, offsets, pages, [n - 1 for n in LENGTHS])
+            out = torch.zeros_like(qd)
+            pool.decode(0, qd, Hq, 1 / math.sqrt(dim), out)
+            ctx.sync()
+            got = out.double().cpu().numpy().reshape(rows, Hq, dim)
+            assert not np.isnan(got).any(), (waves, split)
+            assert np.array_equal(np.where(np.isinf(got), got, 0.0), where), (waves, split)
+    pool.close()
