@@ -25,6 +25,7 @@
 #include "prefill_records.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -526,10 +527,13 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         if constexpr (ROPE)
             k_new = load8<row8>(k_in + in_row).w[0];
 
+        // A state starts at the lowest finite maximum, so that a score of -inf weighs
+        // 2^-inf = 0 also where no other came yet (from -inf it would be NaN), and an
+        // empty state, whose sums are 0, needs no test where states are merged.
         float mx[G], den[G], acc[G][8];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            mx[g] = -INFINITY;
+            mx[g] = -FLT_MAX;
             den[g] = 0.0f;
 #pragma unroll
             for (int f = 0; f < 8; ++f)
@@ -591,7 +595,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                 const float nm = fmaxf(mx[g], fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
                 // rescale only when some lane's running max grew (alpha is 1 elsewhere)
                 if (__builtin_amdgcn_ballot_w64(nm > mx[g])) {
-                    const float alpha = nm == -INFINITY ? 1.0f : fast_exp2(mx[g] - nm);
+                    const float alpha = fast_exp2(mx[g] - nm);
                     den[g] *= alpha;
 #pragma unroll
                     for (int f = 0; f < 8; ++f)
@@ -600,7 +604,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                 }
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    pw[g][j] = ok[j] ? fast_exp2(s[j] - mx[g]) : 0.0f;
+                    pw[g][j] = fast_exp2(s[j] - mx[g]);
                 den[g] += (pw[g][0] + pw[g][1]) + (pw[g][2] + pw[g][3]);
             }
             // token by token: widen the V row once, accumulate it into every q head
@@ -709,7 +713,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
             float M = swap32(mx[g], [](float a, float b) { return fmaxf(a, b); });
             if constexpr (ROWS == 4)
                 M = swap16(M, [](float a, float b) { return fmaxf(a, b); });
-            const float w = mx[g] == -INFINITY ? 0.0f : fast_exp2(mx[g] - M);
+            const float w = fast_exp2(mx[g] - M);
             float d = swap32(den[g] * w, [](float a, float b) { return a + b; });
             if constexpr (ROWS == 4)
                 d = swap16(d, [](float a, float b) { return a + b; });
@@ -744,7 +748,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
         // so that their reads are in flight together (one after another they
         // took half a microsecond).
         auto wg_state = [&](uint32_t n, uint32_t g, uint32_t f, float& M, float& d, float (&a)[4]) {
-            M = -INFINITY;
+            M = -FLT_MAX;
             d = 0.0f;
             a[0] = a[1] = a[2] = a[3] = 0.0f;
             for (uint32_t w0 = 0; w0 < n; w0 += 4) {
@@ -766,12 +770,12 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
 #pragma unroll
                     for (uint32_t i = 1; i < 4; ++i)
                         if (w0 + i >= n) {
-                            ml[i] = make_float2(-INFINITY, 0.0f);
+                            ml[i] = make_float2(-FLT_MAX, 0.0f);
                             av[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                         }
                 }
                 const float nm = fmaxf(fmaxf(M, fmaxf(ml[0].x, ml[1].x)), fmaxf(ml[2].x, ml[3].x));
-                const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
+                const float keep = fast_exp2(M - nm);
                 d *= keep;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -779,7 +783,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                 M = nm;
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i) {
-                    const float weight = ml[i].x == -INFINITY ? 0.0f : fast_exp2(ml[i].x - nm);
+                    const float weight = fast_exp2(ml[i].x - nm);
                     d += ml[i].y * weight;
                     a[0] += av[i].x * weight;
                     a[1] += av[i].y * weight;
@@ -861,7 +865,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
             constexpr uint32_t U = decltype(width)::value;
             for (uint32_t t = tid; t < S * T4; t += blockDim.x) {
                 const uint32_t slice = t / T4, g = t % T4 / (D / 4), f = 4 * t % D;
-                float M = -INFINITY, d = 0.0f, a[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+                float M = -FLT_MAX, d = 0.0f, a[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
                 for (uint32_t c0 = 0; c0 < n_chunks; c0 += U * S) {
                     const uint32_t left = n_chunks - c0; // records from here
                     const __amdgpu_buffer_rsrc_t rec =
@@ -878,10 +882,10 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                     float mc[U], nm = M;
 #pragma unroll
                     for (uint32_t i = 0; i < U; ++i) {
-                        mc[i] = slice + i * S < left ? __uint_as_float(head[i][0]) : -INFINITY;
+                        mc[i] = slice + i * S < left ? __uint_as_float(head[i][0]) : -FLT_MAX;
                         nm = fmaxf(nm, mc[i]);
                     }
-                    const float keep = M == -INFINITY ? 0.0f : fast_exp2(M - nm);
+                    const float keep = fast_exp2(M - nm);
                     d *= keep;
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -889,7 +893,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
                     M = nm;
 #pragma unroll
                     for (uint32_t i = 0; i < U; ++i) {
-                        const float take = slice + i * S < left ? fast_exp2(mc[i] - nm) : 0.0f;
+                        const float take = fast_exp2(mc[i] - nm);
                         d += __uint_as_float(head[i][1]) * take;
 #pragma unroll
                         for (int e = 0; e < 4; ++e)

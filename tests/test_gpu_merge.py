@@ -94,3 +94,51 @@ def test_merges_keep_infinities(ctx, code, dim, group, monkeypatch):
             assert not np.isnan(got).any(), (waves, split)
             assert np.array_equal(np.where(np.isinf(got), got, 0.0), where), (waves, split)
     pool.close()
+
+
+@pytest.mark.parametrize("code,dim,group", [(orc.BF16, 128, 2), (orc.F32, 128, 1), (orc.F16, 256, 4),
+                                            (orc.F32, 256, 2)])
+def test_keys_with_scores_of_minus_infinity_weigh_nothing(ctx, code, dim, group, monkeypatch):
+    """Keys whose product with every query is -inf: the first of a row, single ones,
+    whole pages and a row's last, so that lanes, waves and chunks see no other
+    score (the double reference gives such keys weight 0)."""
+    H, Hq, rows = 2, 2 * group, len(LENGTHS)
+    rng = orc.Mt64(420 + dim + code)
+    pages = [-(-n // 16) for n in LENGTHS]
+    blocks = sum(pages)
+    flat, offsets = rng.permutation(blocks), np.cumsum([0] + pages[:-1])
+    tables = np.split(flat, offsets[1:])
+    positions = [n - 1 for n in LENGTHS]
+    geom, n = (1, blocks, 16, H, dim), blocks * 16 * H * dim
+    kc, vc = rng.normal(n, code), rng.normal(n, code)
+    keys = kc.reshape(-1, H, dim)
+    for r, length in enumerate(LENGTHS[1:], 1):
+        for t in range(length):
+            if t == 0 or t == length - 1 or t % 5 == 3 or 32 <= t < 80:
+                keys[orc.slot(tables[r], t, 16), :, 7] = {orc.F32: -np.inf, orc.BF16: 0xFF80,
+                                                          orc.F16: 0xFC00}[code]
+    q = rng.normal(rows * Hq * dim, code).reshape(rows, Hq, dim)
+    q[:, :, 7] = {orc.F32: 1, orc.BF16: 0x3F80, orc.F16: 0x3C00}[code]
+    q = q.reshape(rows, -1)
+    scale = float(np.float32(1 / math.sqrt(dim)))
+    expected = orc.Attention(geom, kc, vc, code, q, code, positions, flat, offsets, pages, Hq, 0,
+                             scale).reference()
+    assert np.isfinite(expected).all()
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(to_dev(vc, code))
+    qd = to_dev(q, code)
+    for waves in (1, 3, 8):
+        for split in (1, 2, 4, 0):
+            monkeypatch.setenv("CKV_DECODE_WAVES", str(waves))
+            monkeypatch.setenv("CKV_DECODE_SPLIT", str(split))
+            pool.upload(flat, offsets, pages, positions)
+            out = torch.zeros_like(qd)
+            pool.decode(0, qd, Hq, scale, out)
+            ctx.sync()
+            got = to_host(out, code)
+            if code == orc.F32:  # sums of up to 520 terms in another order
+                assert approx(got, expected, 3e-5, 1.0), (waves, split)
+            else:
+                assert_close(orc.to_f32(got, code), expected, what=f"{waves} waves, split {split}")
+    pool.close()
