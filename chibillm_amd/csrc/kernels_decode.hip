@@ -610,8 +610,26 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
             // token by token: widen the V row once, accumulate it into every q head
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
+                // A lane past the row's end re-read the last token: at weight 0 an
+                // infinite value of it would become NaN, so it takes 0. (Selects
+                // in every unit, at most 1 % of a launch: selects in a branch for
+                // the last unit cost 256-wide rows 2.3 % in register copies, a
+                // source of zeros 5.5 % and one long row 6 % in addresses, a copy
+                // of the unit's code spills. f32 words are selected once widened; before,
+                // they spill.)
                 float vf[8];
-                widen8(v[j], vf);
+                row8 vj = v[j];
+                if constexpr (DT != CKV_F32) {
+#pragma unroll
+                    for (uint32_t i = 0; i < row8::words; ++i)
+                        vj.w[i] = ok[j] ? vj.w[i] : make_uint4(0, 0, 0, 0);
+                }
+                widen8(vj, vf);
+                if constexpr (DT == CKV_F32) {
+#pragma unroll
+                    for (int f = 0; f < 8; ++f)
+                        vf[f] = ok[j] ? vf[f] : 0.0f;
+                }
 #pragma unroll
                 for (int g = 0; g < G; ++g)
 #pragma unroll

@@ -142,3 +142,46 @@ def test_keys_with_scores_of_minus_infinity_weigh_nothing(ctx, code, dim, group,
             else:
                 assert_close(orc.to_f32(got, code), expected, what=f"{waves} waves, split {split}")
     pool.close()
+
+
+@pytest.mark.parametrize("code,dim,group,rotary", [
+    (orc.BF16, 256, 4, 64), (orc.F16, 256, 1, None), (orc.F32, 256, 2, None), (orc.BF16, 128, 2, 128),
+    (orc.F16, 128, 8, None), (orc.F32, 128, 4, None)])
+def test_newest_value_row_keeps_infinities(ctx, code, dim, group, rotary):
+    """The newest token's infinities at every position of a page: the lanes past it,
+    which re-read it, make no NaN of them, in the appending call and in a decode
+    of the same pages (there with the queries as they are)."""
+    lengths = list(range(1, 18)) + [47, 48, 200]
+    H, Hq, rows = 2, 2 * group, len(lengths)
+    rng = orc.Mt64(380 + dim + code)
+    pages = [-(-n // 16) for n in lengths]
+    blocks = sum(pages)
+    flat, offsets = rng.permutation(blocks), np.cumsum([0] + pages[:-1])
+    positions = [n - 1 for n in lengths]
+    slots = [orc.slot(t, p, 16) for t, p in zip(np.split(flat, offsets[1:]), positions)]
+    geom, n = (1, blocks, 16, H, dim), blocks * 16 * H * dim
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(rng.normal(n, code), code))
+    vd.copy_(to_dev(rng.normal(n, code), code))
+    qd = to_dev(rng.normal(rows * Hq * dim, code).reshape(rows, -1), code)
+    kn = to_dev(rng.normal(rows * H * dim, code).reshape(rows, -1), code)
+    vn = to_dev(rng.normal(rows * H * dim, code).reshape(rows, H, dim), code)
+    where = np.zeros((rows, Hq, dim))
+    for f, sign in ((0, 1), (5, -1), (dim - 3, 1)):
+        vn[:, :, f] = sign * math.inf
+        where[:, :, f] = sign * np.inf
+    vn, scale = vn.reshape(rows, -1), 1 / math.sqrt(dim)
+    pool.upload(flat, offsets, pages, positions, slots)
+    for again in (False, True):
+        out = torch.zeros_like(qd)
+        if again:
+            pool.decode(0, qd, Hq, scale, out)
+        elif rotary:
+            pool.rope_append_decode(0, kn, vn, qd, Hq, scale, 1e6, out, rotary)
+        else:
+            pool.append_decode(0, kn, vn, qd, Hq, scale, out)
+        ctx.sync()
+        got = out.double().cpu().numpy().reshape(rows, Hq, dim)
+        assert not np.isnan(got).any(), again
+        assert np.array_equal(np.where(np.isinf(got), got, 0.0), where), again
+    pool.close()
