@@ -156,7 +156,7 @@ __device__ __forceinline__ void attend_alone(const uint16_t* __restrict__ keys,
 #pragma unroll
         for (uint32_t j = 0; j < each; ++j) {
             const float other = __shfl_xor(acc[j], d);
-            acc[j] = (keep > 0.0f ? acc[j] * keep : 0.0f) + (w > 0.0f ? other * w : 0.0f);
+            acc[j] = acc[j] * keep + other * w; // a share without keys: 0 at weight 0
         }
     }
     if (sub)

@@ -246,3 +246,41 @@ def test_wide_prefill_keeps_values_that_are_not_finite_with_their_rows(ctx, code
     fin = np.isfinite(general)
     assert_close(got[fin], general[fin], what="finite values")
     assert np.array_equal(np.sign(got[~fin & ~np.isnan(got)]), np.sign(general[~fin & ~np.isnan(general)]))
+
+
+@pytest.mark.parametrize("code,group", [(orc.BF16, 4), (orc.F16, 2)])
+def test_wide_prefill_keeps_nan_of_keys_that_weigh_nothing(ctx, code, group):
+    """0 * NaN and 0 * inf are NaN in the reference: a key whose probability rounds
+    to 0 still passes its NaN on to every query that attends it, as on the general
+    path, however few keys the query attends."""
+    rng = orc.Mt64(1700 + code)
+    H, rows = 2, 40
+    Hq, F, pages = H * group, H * D, 3
+    geom, table = (1, pages, 16, H, D), rng.permutation(pages)
+    k, v = (rng.normal(rows * F, code).reshape(rows, F).copy() for _ in range(2))
+    q = rng.normal(rows * Hq * D, code).reshape(rows, Hq, D)
+    one, low, inf, nan = ((0x3F80, 0xC600, 0x7F80, 0x7FC0) if code == orc.BF16
+                          else (0x3C00, 0xF000, 0x7C00, 0x7E00))
+    q[:, :, 7] = one
+    k[0, 7] = k[0, D + 7] = low  # -8192: a probability of 2^-700 beside any other key's
+    v[0, 3], v[0, D + 9] = nan, inf
+    kc, vc = nan_pages(code, pages * 16 * F), nan_pages(code, pages * 16 * F)
+    orc.store_kv(kc, vc, k, v, [orc.slot(table, p, 16) for p in range(rows)], 0, pages * 16)
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(to_dev(vc, code))
+    pool.upload(table, np.zeros(rows, np.uint32), np.full(rows, pages), np.arange(rows).astype(np.uint32))
+    outs = []
+    for shift in (lambda t: t, misaligned):
+        qd = shift(to_dev(q.reshape(rows, -1), code))
+        out = shift(torch.zeros((rows, Hq * D), dtype=qd.dtype, device="cuda"))
+        pool.attention(0, qd, Hq, 1 / math.sqrt(D), out)
+        ctx.sync()
+        outs.append(orc.to_f32(to_host(out, code), code).reshape(rows, H, group, D))
+    pool.close()
+    got, general = outs
+    assert np.isnan(general[:, 0, :, 3]).all() and np.isnan(general[1:, 1, :, 9]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(general))
+    assert np.array_equal(np.isinf(got), np.isinf(general))
+    fin = np.isfinite(general)
+    assert_close(got[fin], general[fin], what="finite values")
