@@ -38,6 +38,7 @@
 #include "prefill_tile.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cstdlib>
 
 namespace ckv {
@@ -93,82 +94,138 @@ __device__ __forceinline__ void wait_all_but(uint32_t loads)
         __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
-// One query vector against keys 0 .. pos by vector arithmetic: what its wave falls
-// back to when the tile gave it a value that is not finite. A product with
-// P^T multiplies every key of a block for all its queries, so an infinity or NaN
+// Sum over each row of 16 lanes, result in every lane of the row.
+__device__ __forceinline__ float row16_sum(float v)
+{
+    auto add = [&](int moved) { v += __builtin_bit_cast(float, moved); };
+    const auto bits = [&]() { return __builtin_bit_cast(int, v); };
+    add(__builtin_amdgcn_mov_dpp(bits(), 0xB1, 0xF, 0xF, true));  // quad_perm [1,0,3,2]
+    add(__builtin_amdgcn_mov_dpp(bits(), 0x4E, 0xF, 0xF, true));  // quad_perm [2,3,0,1]
+    add(__builtin_amdgcn_mov_dpp(bits(), 0x141, 0xF, 0xF, true)); // row_half_mirror
+    add(__builtin_amdgcn_mov_dpp(bits(), 0x140, 0xF, 0xF, true)); // row_mirror
+    return v;
+}
+
+// Up to alone_queries rows of one query head (bits of `rows`, from row r0 on) against
+// their keys by vector arithmetic: what a wave falls back to for the queries to
+// which the tile gave a value that is not finite. A product with P^T
+// multiplies every key of a block for all its queries, so an infinity or NaN
 // in a V row also meets the zeros of the queries that do not attend it (and of a
 // low term), and 0 * inf is NaN; the decode kernels give such a row only to the
 // queries that attend it, and so does this. Sixteen lanes hold a row, four rows
-// a step; finite results never come here.
+// a step, the next step's in flight; finite results never come here. An infinity
+// early in a shared prefix sends every query of a launch here, so a K/V row read
+// and widened serves several queries: with one in the first page of each
+// sequence the launch below takes 1.81 ms (two at a time 2.29, eight 1.96, one
+// 5.84; the general path took 3.93 for these rows). The cost grows with the
+// rows' positions, as theirs did.
+constexpr uint32_t alone_queries = 4;
+
 template <bool F16>
 __device__ __forceinline__ void attend_alone(const uint16_t* __restrict__ keys,
                                              const uint16_t* __restrict__ values,
                                              const uint32_t* __restrict__ table, uint32_t F,
-                                             uint32_t pos, const uint16_t* q, float c,
-                                             const uint16_t* gate, uint16_t* out, uint32_t lane)
+                                             uint32_t rows, uint32_t pos0, const uint16_t* q,
+                                             size_t q_stride, float c, const uint16_t* gate,
+                                             uint16_t* out, uint32_t lane)
 {
-    constexpr uint32_t each = dim / 16;
+    constexpr uint32_t each = dim / 16, Q = alone_queries;
     const uint32_t f = (lane & 15) * each, sub = lane >> 4;
-    auto features = [](const uint16_t* at, float (&x)[each]) {
-        const u32x4_t w[2] = { reinterpret_cast<const u32x4_t*>(at)[0],
-                               reinterpret_cast<const u32x4_t*>(at)[1] };
+    struct words {
+        u32x4_t w[2];
+    };
+    auto load = [&](const uint16_t* at) {
+        return words { { reinterpret_cast<const u32x4_t*>(at + f)[0],
+                         reinterpret_cast<const u32x4_t*>(at + f)[1] } };
+    };
+    auto widen = [](const words& r, float (&x)[each]) {
 #pragma unroll
         for (uint32_t i = 0; i < each; ++i)
-            x[i] = word_value<F16>(w[i / 8][i / 2 % 4], i % 2);
+            x[i] = word_value<F16>(r.w[i / 8][i / 2 % 4], i % 2);
     };
-    auto weight = [&](float ms, float to) { // 0 for a share that attended nothing
-        return ms == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((ms - to) * c);
+    auto weight = [&](float ms, float to) { return __builtin_amdgcn_exp2f((ms - to) * c); };
+    // the rows (the first again in the places left over) and their states, which
+    // start at the lowest finite maximum: without keys a state weighs 0 or holds 0
+    uint32_t row[Q], count = 0;
+    float qf[Q][each], acc[Q][each], m[Q], l[Q];
+#pragma unroll
+    for (uint32_t i = 0; i < Q; ++i) {
+        row[i] = rows ? __builtin_ctz(rows) : row[0];
+        count += rows != 0;
+        rows &= rows - (rows != 0);
+        widen(load(q + row[i] * q_stride), qf[i]);
+        m[i] = -FLT_MAX;
+        l[i] = 0.0f;
+#pragma unroll
+        for (uint32_t j = 0; j < each; ++j)
+            acc[i][j] = 0.0f;
+    }
+    const uint32_t last = pos0 + row[count - 1]; // the rows ascend
+    uint32_t page = table[0];
+    auto at_key = [&](uint32_t key) { // in the page at hand; past the last key, that one
+        return ((uint64_t)page * page_tokens + min(key, last) % page_tokens) * F;
     };
-    float qf[each], acc[each] = {}, m = -__builtin_inff(), l = 0.0f;
-    features(q + f, qf);
-    for (uint32_t key0 = 0; key0 <= pos; key0 += page_tokens) {
-        const uint64_t page = (uint64_t)table[key0 / page_tokens] * page_tokens;
+    words k_next = load(keys + at_key(sub)), v_next = load(values + at_key(sub));
 #pragma unroll 1
-        for (uint32_t i = 0; i < page_tokens / 4; ++i) {
-            const uint32_t key = key0 + 4 * i + sub;
-            const uint64_t at = (page + min(key, pos) % page_tokens) * F + f;
-            float x[each], s = 0.0f;
-            features(keys + at, x);
+    for (uint32_t key0 = 0; key0 <= last; key0 += 4) {
+        const words k_now = k_next, v_now = v_next;
+        const uint32_t key = key0 + sub, next = key0 + 4;
+        if (next <= last) {
+            if (next % page_tokens == 0)
+                page = table[next / page_tokens];
+            k_next = load(keys + at_key(next + sub));
+            v_next = load(values + at_key(next + sub));
+        }
+        float x[each], s[Q];
+        widen(k_now, x);
+#pragma unroll
+        for (uint32_t i = 0; i < Q; ++i) {
+            s[i] = 0.0f;
 #pragma unroll
             for (uint32_t j = 0; j < each; ++j)
-                s = __builtin_fmaf(qf[j], x[j], s);
+                s[i] = __builtin_fmaf(qf[i][j], x[j], s[i]);
+            s[i] = row16_sum(s[i]);
+        }
+        widen(v_now, x);
 #pragma unroll
-            for (uint32_t d = 1; d < 16; d *= 2)
-                s += __shfl_xor(s, d);
-            features(values + at, x);
-            if (key <= pos) {
-                const float m_new = fmaxf(m, s), keep = weight(m, m_new), w = weight(s, m_new);
-                m = m_new;
-                l = l * keep + w;
+        for (uint32_t i = 0; i < Q; ++i)
+            if (key <= pos0 + row[i]) {
+                const float m_new = fmaxf(m[i], s[i]);
+                const float keep = weight(m[i], m_new), w = weight(s[i], m_new);
+                m[i] = m_new;
+                l[i] = l[i] * keep + w;
 #pragma unroll
                 for (uint32_t j = 0; j < each; ++j)
-                    acc[j] = acc[j] * keep + w * x[j];
+                    acc[i][j] = acc[i][j] * keep + w * x[j];
+            }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < Q; ++i) {
+#pragma unroll
+        for (uint32_t d = 16; d < 64; d *= 2) {
+            const float m_other = __shfl_xor(m[i], d), l_other = __shfl_xor(l[i], d);
+            const float m_new = fmaxf(m[i], m_other);
+            const float keep = weight(m[i], m_new), w = weight(m_other, m_new);
+            m[i] = m_new;
+            l[i] = l[i] * keep + l_other * w;
+#pragma unroll
+            for (uint32_t j = 0; j < each; ++j) {
+                const float other = __shfl_xor(acc[i][j], d);
+                acc[i][j] = acc[i][j] * keep + other * w;
             }
         }
-    }
+        if (i >= count || sub)
+            continue;
+        const float inv = 1.0f / l[i];
+        const size_t at = row[i] * q_stride + f;
 #pragma unroll
-    for (uint32_t d = 16; d < 64; d *= 2) {
-        const float m_other = __shfl_xor(m, d), l_other = __shfl_xor(l, d);
-        const float m_new = fmaxf(m, m_other);
-        const float keep = weight(m, m_new), w = weight(m_other, m_new);
-        m = m_new;
-        l = l * keep + l_other * w;
-#pragma unroll
-        for (uint32_t j = 0; j < each; ++j) {
-            const float other = __shfl_xor(acc[j], d);
-            acc[j] = acc[j] * keep + other * w; // a share without keys: 0 at weight 0
+        for (uint32_t j = 0; j < each; j += 2) {
+            float y[2] = { acc[i][j] * inv, acc[i][j + 1] * inv };
+            if (gate)
+                for (int e = 0; e < 2; ++e)
+                    y[e] *= sigmoid(half_value<F16>(gate[at + j + e]));
+            *reinterpret_cast<uint32_t*>(out + at + j) = pack2<F16>(y[0], y[1]);
         }
-    }
-    if (sub)
-        return;
-    const float inv = 1.0f / l;
-#pragma unroll
-    for (uint32_t j = 0; j < each; j += 2) {
-        float x[2] = { acc[j] * inv, acc[j + 1] * inv };
-        if (gate)
-            for (int e = 0; e < 2; ++e)
-                x[e] *= sigmoid(half_value<F16>(gate[f + j + e]));
-        *reinterpret_cast<uint32_t*>(out + f + j) = pack2<F16>(x[0], x[1]);
     }
 }
 
@@ -612,12 +669,19 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
                     make_uint2(pack2<F16>(x[0], x[1]), pack2<F16>(x[2], x[3]));
             }
     }
-    for (uint32_t left = alone; left; left &= left - 1) {
-        const uint32_t r = rb * 32 + __builtin_ctz(left);
-        const size_t at = (size_t)(row0 + r) * q_stride + (size_t)head * dim;
+    if (__builtin_expect(alone == 0, 1)) // (62.4 us; with the loop in its place 63.3)
+        return;
+    const size_t first = (size_t)(row0 + rb * 32) * q_stride + (size_t)head * dim;
+    for (uint32_t left = alone; left;) {
+        uint32_t some = left; // the lowest alone_queries of them
+#pragma unroll
+        for (uint32_t i = 0; i < alone_queries; ++i)
+            left &= left - 1;
+        some ^= left;
         attend_alone<F16>(static_cast<const uint16_t*>(p.keys) + base_elems,
-                          static_cast<const uint16_t*>(p.values) + base_elems, table, F, pos0 + r,
-                          q + at, c, gate ? gate + at : nullptr, out + at, lane);
+                          static_cast<const uint16_t*>(p.values) + base_elems, table, F, some,
+                          pos_lo, q + first, q_stride, c, gate ? gate + first : nullptr,
+                          out + first, lane);
     }
 }
 

@@ -284,3 +284,46 @@ def test_wide_prefill_keeps_nan_of_keys_that_weigh_nothing(ctx, code, group):
     assert np.array_equal(np.isinf(got), np.isinf(general))
     fin = np.isfinite(general)
     assert_close(got[fin], general[fin], what="finite values")
+
+
+@pytest.mark.parametrize("code,group", [(orc.BF16, 4), (orc.F16, 8)])
+def test_wide_prefill_with_an_infinity_early_in_a_prefix(ctx, code, group):
+    """Every query of the launch attends an infinite value and is attended again by
+    vector arithmetic, several at a time: the counts of such queries in a wave
+    run over 1 to 32, and all values but the infinite ones stay those of the
+    double reference."""
+    rng = orc.Mt64(1800 + code)
+    H, chunks = 1, [(19, n) for n in (1, 2, 3, 4, 5, 31, 32, 33, 70)]
+    Hq, F = H * group, H * D
+    spans = [p + n for p, n in chunks]
+    pages = [-(-n // 16) for n in spans]
+    blocks = sum(pages)
+    tables = np.split(rng.permutation(blocks), np.cumsum(pages)[:-1])
+    seq = np.repeat(np.arange(len(chunks)), [n for _, n in chunks])
+    positions = np.concatenate([np.arange(p, p + n) for p, n in chunks]).astype(np.uint32)
+    flat, offsets = np.concatenate(tables), np.cumsum([0] + pages[:-1])[seq]
+    lengths, rows, geom = np.array(pages)[seq], len(positions), (1, blocks, 16, H, D)
+    kc, vc = nan_pages(code, blocks * 16 * F), nan_pages(code, blocks * 16 * F)
+    for t, n in zip(tables, spans):
+        orc.store_kv(kc, vc, rng.normal(n * F, code).reshape(-1, F), rng.normal(n * F, code).reshape(-1, F),
+                     [orc.slot(t, p, 16) for p in range(n)], 0, blocks * 16)
+    q = rng.normal(rows * Hq * D, code).reshape(rows, -1)
+    scale = float(np.float32(1 / math.sqrt(D)))
+    expected = orc.Attention(geom, kc, vc, code, q, code, positions, flat, offsets, lengths, Hq, 0,
+                             scale).reference().reshape(rows, Hq, D).copy()
+    expected[:, :, 17] = np.inf
+    for t in tables:
+        vc.reshape(-1, F)[orc.slot(t, 2, 16), 17] = 0x7F80 if code == orc.BF16 else 0x7C00
+    pool, kd, vd = new_pool(ctx, geom, code)
+    kd.copy_(to_dev(kc, code))
+    vd.copy_(to_dev(vc, code))
+    pool.upload(flat, offsets, lengths, positions)
+    qd = to_dev(q, code)
+    out = torch.full_like(qd, float("nan"))
+    pool.attention(0, qd, Hq, scale, out)
+    ctx.sync()
+    got = orc.to_f32(to_host(out, code), code).reshape(rows, Hq, D)
+    pool.close()
+    assert np.array_equal(got[:, :, 17], expected[:, :, 17])
+    others = np.arange(D) != 17
+    assert_close(got[:, :, others], expected[:, :, others], what="finite values")
