@@ -136,7 +136,7 @@ CHUNKS = [(0, 1), (0, 33), (5, 40), (31, 64), (100, 128), (16, 257), (700, 1), (
 def test_wide_prefill_matches_oracle_and_general_path(ctx, code, group, gated, split, min_blocks,
                                                       monkeypatch):
     """Tiles on the matrix cores (f32 pools: decode rows) with keys unsplit and
-    split. Probabilities enter as two 16-bit terms, so the error against the
+    split. Probabilities enter as three 16-bit terms, so the error against the
     double reference is that of the general path, which holds them in 32 bits:
     both round the same stored values once (bounded at 1.1 times here, for the
     order of sums)."""
@@ -327,3 +327,41 @@ def test_wide_prefill_with_an_infinity_early_in_a_prefix(ctx, code, group):
     assert np.array_equal(got[:, :, 17], expected[:, :, 17])
     others = np.arange(D) != 17
     assert_close(got[:, :, others], expected[:, :, others], what="finite values")
+
+
+@pytest.mark.parametrize("code", [orc.BF16, orc.F16])
+def test_wide_prefill_holds_probabilities_in_32_bits(ctx, code):
+    """Values that cancel show a probability's own rounding. In each sequence of
+    four tokens the first key has probability p = e^(-y / 16) beside three of 1,
+    whose values are the parts of -p in the 16-bit type: the last row's output
+    is what p's roundings leave, over 3 + p > 3.3. Bound: p off by 2^-22 (its
+    exponent's two roundings and the exponential's last place), its parts by 2^-24,
+    and six matrix products rounding sums of at most 1 twice, 12 * 2^-24: 3e-7, plus
+    half of fp16's smallest value. (bf16 probabilities in two terms, 16 bits, leave
+    up to 1e-6 for half of these y.)"""
+    H, group, n, count = 1, 4, 4, 64
+    to = torch.bfloat16 if code == orc.BF16 else torch.float16
+    y = torch.arange(1, count + 1, dtype=torch.float64) / 4
+    k, v = (torch.zeros(count, 16, D, dtype=torch.float64) for _ in range(2))
+    k[:, 0, 0] = -y
+    v[:, 0] = 1.0
+    left = -torch.exp(-y / 16)
+    for part in (1, 2, 3):
+        v[:, part] = left.to(to).double()[:, None]
+        left = left - v[:, part, 0]
+    q = torch.zeros(count, n, group, D, dtype=torch.float64)
+    q[..., 0] = 1.0
+    order = torch.arange(count - 1, -1, -1)  # sequence i on page count - 1 - i
+    pool, kd, vd = new_pool(ctx, (1, count, 16, H, D), code)
+    kd.copy_(k[order].to(to).reshape(-1).cuda())
+    vd.copy_(v[order].to(to).reshape(-1).cuda())
+    rows = count * n
+    pool.upload(order.numpy().astype(np.uint32), np.repeat(np.arange(count), n), np.ones(rows, np.uint32),
+                np.tile(np.arange(n), count).astype(np.uint32))
+    qd = q.reshape(rows, -1).to(to).cuda()
+    out = torch.full_like(qd, float("nan"))
+    pool.attention(0, qd, group, 1 / 16, out)
+    ctx.sync()
+    pool.close()
+    last = out.double().cpu().reshape(count, n, group, D)[:, -1]
+    assert last.abs().max() <= 3e-7 + 2.0 ** -25, float(last.abs().max())
