@@ -452,6 +452,56 @@ TEST("prefill launch shape: small launches take 4-wave workgroups and split keys
     CHECK(prefill_shape_for(8, 8, 16, 256, CKV_BF16, 500).waves == 4);
 }
 
+TEST("prefill launch shape of 256-wide heads: ranges that fill the compute units, records for all")
+{
+    // tiles of `rows` rows each, as the uploads count them
+    auto plan_of = [](uint32_t n_tiles, uint32_t rows, uint32_t kv_heads, uint32_t group, int cus) {
+        ckv::pool_view p {};
+        p.kv_heads = kv_heads;
+        p.head_dim = 256;
+        p.block_size = 16;
+        p.features = kv_heads * 256;
+        p.dtype = CKV_F16;
+        ckv::meta_view m {};
+        m.n_tiles = n_tiles;
+        m.tile_blocks = 75;
+        for (uint32_t i = 0; i < 3; ++i)
+            m.row_blocks[i] = n_tiles * ((rows + (32u << i) - 1) / (32u << i));
+        return ckv::prefill_plan(p, m, group * kv_heads, cus);
+    };
+    for (const uint32_t group : { 1u, 2u, 4u, 8u })
+        for (const uint32_t kv_heads : { 1u, 2u, 4u, 16u })
+            for (const uint32_t n_tiles : { 1u, 3u, 8u, 64u, 500u })
+                for (const uint32_t rows : { 2u, 33u, 130u, 256u })
+                    for (const char* forced : { "", "1", "3", "50" }) {
+                        const env_guard e(*forced ? "CKV_PREFILL_SPLIT" : "CKV_UNUSED", forced);
+                        const auto s = plan_of(n_tiles, rows, kv_heads, group, 256);
+                        // the kernel's workgroups: 128 / G rows of a tile and G heads each
+                        const uint64_t G = std::min(group, 4u), subs = 256 / (128 / G);
+                        const uint64_t pairs = n_tiles * subs * (group / G) * kv_heads;
+                        const uint64_t busy = (uint64_t)n_tiles * ((rows + 128 / G - 1) / (128 / G))
+                            * (group / G) * kv_heads;
+                        // a record: 65 chunks of four floats per query vector, 128 to a workgroup
+                        const uint64_t record = 65 * 4 * 128, room = (128ull << 20) / 4;
+                        REQUIRE(s.waves == 4 && s.n_split >= 1 && s.n_split <= ckv::split_max);
+                        if (s.n_split > 1) {
+                            CHECK(s.counters == pairs);
+                            CHECK(s.records_floats == pairs * s.n_split * record);
+                            CHECK(s.records_floats <= room);
+                        } else {
+                            CHECK(s.counters == 0 && s.records_floats == 0);
+                        }
+                        const uint64_t want = *forced ? (uint64_t)std::atoi(forced) : 256 / busy;
+                        const uint64_t fits = std::max<uint64_t>(1, room / (pairs * record));
+                        CHECK(s.n_split == std::clamp<uint64_t>(std::min(want, fits), 1, ckv::split_max));
+                    }
+    // four sequences of about 400 rows in two tiles each, groups of four over two kv heads
+    CHECK(plan_of(8, 200, 2, 4, 256).n_split == 2);
+    // 64 tiles of two rows: records for 512 workgroups, 448 of them past their
+    // tile's rows, so a second range has no room
+    CHECK(plan_of(64, 2, 1, 4, 256).n_split == 1);
+}
+
 TEST("prefill launch shape: the environment overrides")
 {
     {

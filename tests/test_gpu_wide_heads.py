@@ -365,3 +365,43 @@ def test_wide_prefill_holds_probabilities_in_32_bits(ctx, code):
     pool.close()
     last = out.double().cpu().reshape(count, n, group, D)[:, -1]
     assert last.abs().max() <= 3e-7 + 2.0 ** -25, float(last.abs().max())
+
+
+@pytest.mark.parametrize("code,split", [(orc.BF16, "1"), (orc.F16, "3")])
+def test_wide_heads_in_a_layer_past_4_gib(ctx, code, split, monkeypatch):
+    """A layer of 140,000 pages of 32 KiB (4.3 GiB per tensor): pages above the
+    4 GiB line, alone and among low ones, in prefill and decode."""
+    monkeypatch.setenv("CKV_PREFILL_SPLIT", split)
+    monkeypatch.setenv("CKV_PREFILL_SPLIT_MIN", "1")
+    rng = orc.Mt64(2000 + code)
+    H, group, n, chunk, blocks = 4, 2, 210, 70, 140_000
+    Hq, F, pages = H * group, H * D, 14
+    assert blocks * 16 * F * 2 > 1 << 32
+    print(f"256-wide heads over {blocks} pages, dtype {code} split {split}", flush=True)
+    high = np.arange(blocks - pages, blocks, dtype=np.uint32)
+    mixed = np.where(np.arange(pages) % 2, blocks - 40 + np.arange(pages), 5 + np.arange(pages)).astype(np.uint32)
+    tables = [high, mixed]
+    k, v = (rng.normal(2 * n * F, code).reshape(2, n, F) for _ in range(2))
+    q = rng.normal(2 * chunk * Hq * D, code).reshape(2 * chunk, -1)
+    kc, vc = (np.zeros(2 * pages * 16 * F, np.uint16) for _ in range(2))
+    pool, _, _ = new_pool(ctx, (1, blocks, 16, H, D), code)
+    for i, t in enumerate(tables):
+        pool.upload(t, [0] * n, [pages] * n, list(range(n)), [orc.slot(t, p, 16) for p in range(n)])
+        pool.append(0, to_dev(k[i], code), to_dev(v[i], code))
+        compact = np.arange(i * pages, (i + 1) * pages, dtype=np.uint32)
+        orc.store_kv(kc, vc, k[i], v[i], [orc.slot(compact, p, 16) for p in range(n)], 0, 2 * pages * 16)
+    positions = list(range(n - chunk, n)) * 2
+    offsets, lengths = [0] * chunk + [pages] * chunk, [pages] * (2 * chunk)
+    scale = float(np.float32(1 / math.sqrt(D)))
+    expected = orc.Attention((1, 2 * pages, 16, H, D), kc, vc, code, q, code, positions,
+                             np.arange(2 * pages, dtype=np.uint32), offsets, lengths, Hq, 0, scale).reference()
+    pool.upload(np.concatenate(tables), offsets, lengths, positions)
+    qd = to_dev(q, code)
+    for name in ("attention", "decode"):
+        out = torch.full_like(qd, float("nan"))
+        getattr(pool, name)(0, qd, Hq, scale, out)
+        ctx.sync()
+        assert_close(orc.to_f32(to_host(out, code), code), expected, what=name)
+    pool.close()
+    del pool
+    torch.cuda.empty_cache()
