@@ -297,6 +297,21 @@ TEST("small batches: chunks that fit one round of workgroups")
     }
 }
 
+TEST("more than two units per compute unit: whole rows only where they even out")
+{
+    auto whole = [](uint32_t rows, uint32_t low, uint32_t high) {
+        std::vector<uint32_t> p(rows);
+        for (uint32_t i = 0; i < rows; ++i) // evenly spread lengths
+            p[i] = low + (uint32_t)((uint64_t)(high - low) * i / (rows - 1)) - 1;
+        return plan_and_check(p, 8, 256).shape.n_cut == 0;
+    };
+    // short rows fill the last round: the fullest of 32 sets of compute units holds
+    // 1.10 and 1.12 times its share
+    CHECK(whole(96, 100, 3000) && whole(80, 100, 3000));
+    // nearly equal rows, two rounds and a part of a third: 1.22, 1.33 and 1.29 times
+    CHECK(!whole(72, 1000, 2500) && !whole(70, 2290, 2983) && !whole(73, 160, 216));
+}
+
 TEST("random batches at random GPU sizes: every plan is well formed")
 {
     std::mt19937_64 g(7);
