@@ -1012,9 +1012,10 @@ constexpr uint32_t split_alone_min_pages = 48;
 constexpr uint32_t split_uncut_slack = 47;
 // How a pool's decode fills the GPU (decode_form). 16-bit pages of 128-wide
 // heads: two 8-wave workgroups per compute unit. f32 pages: two of 4 waves; a
-// whole row on 4 waves reads at a fraction of a compute unit's rate, so rows are
-// not kept whole for want of balance alone (48 rows of U[256, 4096] tokens whole
-// 170 us, dealt out 130). 256-wide heads: one workgroup of 8 waves (with more
+// whole row on 4 waves reads at a fraction of a compute unit's rate, so rows stay
+// whole only while none is over 9/8 of the share and they even out (whole_rows_even):
+// 48 rows of U[256, 700] tokens, longest 0.96 times the share, cut 39.0 us, whole 35.7;
+// 36 of U[400, 900], 1.24 times, 35.1 and 41.4; 48 of U[256, 4096], 1.25, 130 and 170. 256-wide heads: one workgroup of 8 waves (with more
 // than two q heads per kv head its lanes need the registers of two); a page is
 // twice the bytes, so chunks may be shorter and the slack is half.
 constexpr decode_form form_narrow { 2, 12, 32, split_uncut_slack, false };
@@ -1421,15 +1422,20 @@ uint64_t small_batch_span(const std::vector<uint32_t>& positions, uint32_t block
 }
 
 // Whether whole rows, started longest first on the compute unit that is free
-// first, leave none with more than 6/5 of its share of the pages. Measured on
+// first, leave none with more than num/den of its share of the pages. Measured on
 // MI355X (16-bit pages, 8 kv heads, 65 to 112 rows) against chunks of a quarter
 // of the share: at 1.10 to 1.15 times the share whole rows are 1 to 4 % faster
 // (96 rows of U[100, 3000] tokens 100.2 and 103.5 us, 80 rows 86.5 and 87.9), near 1.2 the
 // two tie (74 rows of U[784, 2096] 81.7 and 81.9), and past it chunks are: 72 rows
 // of U[1000, 2500] (1.22) 89.4 and 93.0, 70 of U[2290, 2983] (1.33) 133 and 140, 73 of
-// U[160, 216] (1.29) 17.6 and 18.3.
+// U[160, 216] (1.29) 17.6 and 18.3. f32 rows of one or two units per compute unit,
+// against their cut plan: up to 1.17 whole rows are 2 to 13 % faster (64 rows of
+// U[764, 1286], 1.01: 88.8 and 98.6; but 64 of U[245, 1833], 1.00, 95.6 and 87.0), between
+// 1.2 and 1.25 they gain 20 % or lose 3 to 5 % (42 of U[276, 623] 32.0 and 39.8, 49
+// of U[741, 1239] 70.1 and 66.6), past that they mostly lose (38 of U[1008, 1153], 1.61,
+// 62.3 and 56.3).
 bool whole_rows_even(const std::vector<uint32_t>& positions, uint32_t block_size, uint32_t kv_heads,
-                     uint64_t cus, uint64_t total)
+                     uint64_t cus, uint64_t total, uint64_t num, uint64_t den)
 {
     std::vector<uint64_t> pages(positions.size());
     std::transform(positions.begin(), positions.end(), pages.begin(),
@@ -1443,7 +1449,7 @@ bool whole_rows_even(const std::vector<uint32_t>& positions, uint32_t block_size
         load.back() += n;
         std::push_heap(load.begin(), load.end(), std::greater<> {});
     }
-    return 5 * sets * *std::max_element(load.begin(), load.end()) <= 6 * total;
+    return den * sets * *std::max_element(load.begin(), load.end()) <= num * total;
 }
 
 uint64_t forced_pages(const char* name, bool& set)
@@ -1490,17 +1496,22 @@ decode_plan_shape shape_decode_plan(const std::vector<uint32_t>& positions, uint
         // share: a cut costs its merge and second segment, and the cut plan's
         // pages run about 12 % slower than a whole row's. With more units per
         // compute unit the fixed chunks balance better (the config-5 churn's
-        // batches of hundreds of rows: 1.5 % faster cut).
+        // batches of hundreds of rows: 1.5 % faster cut), unless whole rows,
+        // which start longest first, even out.
         const uint64_t units = (uint64_t)rows * kv_heads;
-        const bool fill = !form.few_waves && units >= cus && units <= 2 * cus;
-        const uint64_t slack = std::min(share / 8 + form.uncut_slack, 5 * share / 8);
-        // with more than two units per compute unit, whole rows start longest
-        // first and may even out (whole_rows_even)
-        const auto even = [&]() {
-            return units > 2 * cus && 5 * longest <= 4 * share
-                && whole_rows_even(positions, block_size, kv_heads, cus, total);
+        const auto whole = [&]() {
+            const auto even = [&](uint64_t num, uint64_t den) {
+                return whole_rows_even(positions, block_size, kv_heads, cus, total, num, den);
+            };
+            if (units > 2 * cus)
+                return 5 * longest <= 4 * share && even(6, 5);
+            if (units < cus)
+                return false;
+            return form.few_waves
+                ? longest <= share + share / 8 && even(5, 4)
+                : longest <= share + std::min(share / 8 + form.uncut_slack, 5 * share / 8);
         };
-        if (2 * longest > share && !even() && (!fill || longest > share + slack)) {
+        if (2 * longest > share && !whole()) {
             // as many workgroups as the GPU holds at once, but no more than a
             // row each where rows are short (pieces of at least
             // split_min_pages), nor more than max_chunks to a row

@@ -312,6 +312,22 @@ TEST("more than two units per compute unit: whole rows only where they even out"
     CHECK(!whole(72, 1000, 2500) && !whole(70, 2290, 2983) && !whole(73, 160, 216));
 }
 
+TEST("f32 pages: rows stay whole while none is over 9/8 of a compute unit's share and they even out")
+{
+    auto whole = [](uint32_t rows, uint32_t low, uint32_t high) {
+        std::vector<uint32_t> p(rows);
+        for (uint32_t i = 0; i < rows; ++i)
+            p[i] = low + (uint32_t)((uint64_t)(high - low) * i / (rows - 1)) - 1;
+        return plan_and_check(p, 8, 256, ckv::decode_form_of(CKV_F32, 128)).shape.n_cut == 0;
+    };
+    // the fullest set of compute units holds 1.00, 1.05 and 1.23 times its share
+    CHECK(whole(64, 764, 1286) && whole(61, 125, 340) && whole(42, 276, 623));
+    CHECK(whole(32, 512, 512));
+    CHECK(!whole(38, 1008, 1153) && !whole(44, 2260, 2486)); // 1.6 and 1.4 times
+    CHECK(!whole(36, 400, 900) && !whole(40, 100, 600) && !whole(48, 256, 4096)); // longer
+    CHECK(!whole(31, 512, 512)); // fewer units than compute units
+}
+
 TEST("random batches at random GPU sizes: every plan is well formed")
 {
     std::mt19937_64 g(7);
