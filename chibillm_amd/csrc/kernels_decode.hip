@@ -1368,8 +1368,9 @@ uint64_t balanced_work(const std::vector<uint32_t>& positions, uint32_t block_si
 
 // Chunk length, in pages, of a batch too small to deal out page by page, or 0
 // when it is better dealt out all the same. The times of three plans are
-// weighed in pages of one workgroup alone on its compute unit (k workgroups
-// there share its reads, so a page takes each k times as long): the shortest
+// weighed in tenths of a page of one workgroup alone on its compute unit (k
+// workgroups there share its reads, so a page takes each k times as long; two of
+// the f32 form's, too small to read at the full rate, 1.6 times): the shortest
 // chunks that make at most k workgroups per compute unit take span * k for each
 // k, and the balanced plan its pages and, for each row, the round trips of one
 // more segment. Rows whose chunks fit one round of workgroups end together;
@@ -1390,6 +1391,7 @@ uint64_t small_batch_span(const std::vector<uint32_t>& positions, uint32_t block
     const uint64_t shortest = std::max<uint64_t>(
         { form.min_pages, (longest + form.max_chunks - 1) / form.max_chunks,
           (uint64_t)std::sqrt((double)longest / 8) });
+    const auto tenths = [&](uint64_t k) { return form.few_waves && k == 2 ? 16 : 10 * k; };
     uint64_t best_span = 0, best = UINT64_MAX;
     uint64_t slots = 1;
     for (uint64_t k = 1; k <= form.per_cu; ++k) {
@@ -1408,15 +1410,21 @@ uint64_t small_batch_span(const std::vector<uint32_t>& positions, uint32_t block
             else
                 lo = mid + 1;
         }
-        if (hi * k < best || (form.few_waves && hi * k == best)) {
-            best = hi * k;
+        if (hi * tenths(k) < best) {
+            best = hi * tenths(k);
             best_span = hi;
         }
     }
-    // pages of work the balanced plan gives a compute unit
-    const uint64_t work = form.per_cu * (total + split_row_pages / form.per_cu * rows);
-    const uint64_t dealt = (work + slots - 1) / slots;
-    if (total >= slots * form.min_pages && rows <= slots && 100 * dealt < 97 * best)
+    // Work the balanced plan gives a compute unit, and the line below which it is
+    // taken. Measured at dealt over best, dealt against chunks, us: 16-bit 0.84 (30
+    // rows of U[100, 2000] tokens) 26.3 and 27.6, 0.92 (14 of U[100, 4000]) 24.3 and 25.2,
+    // 0.95 (8 of U[3000, 4100]) 23.6 and 25.0, 0.96 (12 of U[500, 3000]) 19.0 and 19.8, 1.06 (16
+    // of 1,000) 17.0 and 15.4; f32 0.87 (24 of U[100, 2500]) 43.9 and 45.8, 0.92 (14 of
+    // U[100, 4000]) 40.4 and 41.7, 0.93 (16 of U[200, 2000]) 28.5 and 26.7, 0.94 (20 of U[1000,
+    // 1300]) 36.1 and 34.0.
+    const uint64_t work = tenths(form.per_cu) * (total + split_row_pages / form.per_cu * rows);
+    const uint64_t dealt = (work + slots - 1) / slots, line = form.few_waves ? 92 : 97;
+    if (total >= slots * form.min_pages && rows <= slots && 100 * dealt < line * best)
         return 0;
     return best_span;
 }
