@@ -394,13 +394,14 @@ __device__ __forceinline__ void store_elem(void* base, uint64_t i, float x)
 // current page is processed. Lane 16*group + part reads features 8*part..8*part+7 of token
 // 4j + group of the page (j = 0..3): four 1 KiB wave loads per page for K and
 // four for V (256-wide heads: lane 32*group + part, token 2j + group of half a
-// page; pages below stand for these units). The wave's four row-group softmax states are merged with
-// shuffles, the W wave states through LDS, and the workgroup writes the
-// normalised output of the group's q heads. GATED multiplies it by
-// sigmoid(gate) first; the gate values are loaded when the workgroup starts,
-// so their latency hides behind the page loads. A chunk of a cut row writes
-// its unnormalised state instead (a partial record per q head) with
-// agent-scope stores and counts itself in; the chunk that arrives last merges
+// page; pages below stand for these units). The wave's row-group softmax states
+// are reduced and scattered by lane swaps, the W wave states merged through
+// LDS, and the workgroup writes the normalised output of the group's q heads.
+// GATED multiplies it by sigmoid(gate) first; the gate values are loaded after
+// the last page, into its registers, so that their latency hides behind the
+// merge. A chunk of a cut row writes its unnormalised state instead (a partial
+// record per q head) with 16-byte write-through stores (prefill_records.h) and
+// counts itself in; the chunk that arrives last merges
 // the row's records in the same launch. (An agent-scope release fence per
 // workgroup would write back the XCD's whole L2, measured at about 1.9 us per
 // workgroup per XCD; stores that are coherent on their own need only a wait
@@ -1000,24 +1001,30 @@ constexpr uint32_t split_waves_alone = 12;
 constexpr uint32_t split_alone_min_pages = 48;
 // Pages (about 12 us of one workgroup's reads) by which the longest row may
 // exceed 9/8 of a compute unit's share and still stay whole, for batches of
-// one or two (row, kv head) units per compute unit (and no more than 13/8 of
-// the share: 32 rows of U[300, 2000] tokens, longest 1.73 times the share, cut
-// 31.7 us, whole 34.5). Measured on one
-// MI355X layer (fused, bf16, 8 kv heads) against cutting: 32 rows of
-// U[512, 1536] tokens -15 %, U[768, 1280] -9 %, 1,024 tokens -7 %, 2,048 -6 %,
-// 64 rows of U[64, 2048] -5 %, 48 rows of U[256, 4096] -3.5 %; config 2's 32
-// rows of U[256, 4096] (longest 256 pages, share 144) still cut, as do batches
-// of fewer (row, kv head) units than compute units (8 rows of 1,024 tokens
-// whole: +36 %).
+// one or two (row, kv head) units per compute unit, and no more than 13/8 of
+// the share. Measured on one MI355X layer (fused, bf16, 8 kv heads), longest over
+// share, whole and dealt out, us: 48 rows of U[200, 2000] tokens 1.21, 39.2 and
+// 39.7; 56 of U[200, 2400] 1.06, 50.9 and 52.4; 64 of U[300, 3000] 0.91, 70.4 and 73.1; 36
+// of U[100, 1200] 1.63, 23.6 and 21.7; 32 of U[300, 2000] 1.74, 36.5 and 30.6; 32 of
+// U[1000, 3500] 1.55 (61 pages over), 60.2 and 51.5. Between 1.3 and the cap cutting
+// has become the faster with its cheaper merges (32 of U[500, 1500] 1.49, 29.7
+// and 27.2; 40 of U[300, 2000] 1.39, 37.7 and 35.2; 32 of U[400, 1700] 1.62, 32.2 and
+// 28.5), which the line does not follow yet. Batches of fewer (row, kv head)
+// units than compute units are cut (8 rows of 1,024 tokens whole: +36 %).
 constexpr uint32_t split_uncut_slack = 47;
 // How a pool's decode fills the GPU (decode_form). 16-bit pages of 128-wide
 // heads: two 8-wave workgroups per compute unit. f32 pages: two of 4 waves; a
 // whole row on 4 waves reads at a fraction of a compute unit's rate, so rows stay
 // whole only while none is over 9/8 of the share and they even out (whole_rows_even):
 // 48 rows of U[256, 700] tokens, longest 0.96 times the share, cut 39.0 us, whole 35.7;
-// 36 of U[400, 900], 1.24 times, 35.1 and 41.4; 48 of U[256, 4096], 1.25, 130 and 170. 256-wide heads: one workgroup of 8 waves (with more
-// than two q heads per kv head its lanes need the registers of two); a page is
-// twice the bytes, so chunks may be shorter and the slack is half.
+// 36 of U[400, 900], 1.24 times, 35.1 and 41.4; 48 of U[256, 4096], 1.25, 130 and 170.
+// 256-wide heads: one workgroup of 8 waves. With more than two q heads per kv
+// head its lanes need the registers of two; with one or two, two would fit, but
+// a plan for two is slower (2 kv heads, chunks for one and for two workgroups
+// per compute unit, us: 32 rows of U[256, 4096] tokens 27.0 and 29.6 at one q head
+// per kv head, 28.5 and 32.0 at two; 32 of 1,000 14.7 and 15.0, 16.0 and 16.3; 16 of
+// U[100, 2500] 12.0 and 13.7, 13.2 and 15.1). A page is twice the bytes, so chunks may
+// be shorter and the slack is half.
 constexpr decode_form form_narrow { 2, 12, 32, split_uncut_slack, false };
 constexpr decode_form form_f32 { 2, 8, 32, 0, true };
 constexpr decode_form form_wide { 1, 4, 128, split_uncut_slack / 2, false };
@@ -1522,7 +1529,7 @@ decode_plan_shape shape_decode_plan(const std::vector<uint32_t>& positions, uint
         if (2 * longest > share && !whole()) {
             // as many workgroups as the GPU holds at once, but no more than a
             // row each where rows are short (pieces of at least
-            // split_min_pages), nor more than max_chunks to a row
+            // form.min_pages), nor more than max_chunks to a row
             const uint64_t slots = std::max<uint64_t>(1, cus * form.per_cu / kv_heads);
             const uint64_t piece = std::max<uint64_t>(
                 form.min_pages, (longest + form.max_chunks - 1) / form.max_chunks);

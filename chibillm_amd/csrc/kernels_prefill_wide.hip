@@ -25,18 +25,22 @@
 // vector ALU forms the probabilities of block kb - 1 and V(kb - 1) is read;
 // then O^T of block kb - 1 is multiplied while K(kb + 1) is read and the scores
 // of block kb are masked and searched for maxima. K has to be staged one block
-// sooner than V: K and V have four LDS stages each (131 KB, one workgroup per
+// sooner than V: K and V have four LDS stages each (132 KiB, one workgroup per
 // compute unit), iteration kb loads K(kb + 3) and V(kb + 2), and its barrier
 // publishes K(kb + 2) and V(kb).
 //
 // Four sequences of 300 to 512 rows behind 700 tokens (2 kv heads, 8 q heads,
-// gated) take 50 us for 12.1 GFLOP, where the same rows through the decode
-// kernel took 440: 102 workgroups, their keys in two ranges, so the longest runs
-// 23 blocks one after another. A block takes 3,500 cycles of a wave: 1,000 to
-// issue its loads (about 32 bytes a cycle and compute unit pass to LDS), 890 for
-// the scores and probabilities, 720 for P.V, 700 for maxima, waits and rescales.
-// Issuing the loads in twos between those phases took 64.1 to 64.7 us in all
-// instead of 62.3; reading both halves of V before the scores 64.7.
+// gated, 12.1 GFLOP) take 66.7 us with their two rotations, of them 61.6 here (in
+// a kernel trace; the general path took 3,900 to 4,100): 104 workgroups of 32 rows, of which the
+// eight that start a sequence, 23 key blocks each, are not cut (fewer than three ranges'
+// worth of blocks) and the others have their 24 to 38 blocks in two ranges. The
+// uncut ones are the longest chains, and what bounds the launch is such a chain, not
+// the matrix cores. With two-term probabilities a block took 3,500 cycles of a wave:
+// 1,000 to issue its loads (about 32 bytes a cycle and compute unit pass to LDS), 890
+// for the scores and probabilities, 720 for P.V, 700 for maxima, waits and
+// rescales; the third term adds about 480. Issuing the loads in twos between those
+// phases took 64.1 to 64.7 us in all instead of 62.3; reading both halves of V
+// before the scores 64.7.
 #include "ckv_internal.h"
 #include "prefill_records.h"
 #include "prefill_tile.h"
@@ -60,8 +64,8 @@ constexpr uint32_t tiles_o = dim / 32; // accumulators of O^T
 // row k in the order chunk ^ (k % 16): a DMA instruction moves two whole rows
 // (eight full cache lines), and the 16 lanes that read a chunk of 16 rows
 // together find it at 16 different bank offsets (staged in operand order, 32 bytes
-// of each of 32 rows per instruction, the launch below took 62.9 us instead of
-// 62.3).
+// of each of 32 rows per instruction, that launch took 62.9 us instead of
+// 62.3, with its rotations and two-term probabilities).
 constexpr uint32_t k_stage_bytes = block_keys * dim * 2;
 // V stage: two halves of 128 features, each as kernels_prefill.hip stages a
 // 128-wide head: 8 groups of 4 key rows, 64 bytes after each group.
@@ -405,7 +409,7 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
                 va[mt][h] = make_uint4(l2.x, l2.y, h2.x, h2.y);
             }
     };
-    // the probabilities of sp as two 16-bit terms, and their share of the denominator
+    // the probabilities of sp as 16-bit terms, and their share of the denominator
     auto probabilities = [&](uint4 (&pt)[terms][2]) {
         // a range of the keys may hold none a query attends yet (m = -inf)
         const float bias = F16 ? p_scale_f16 : 0.0f;
@@ -715,7 +719,7 @@ hipError_t launch_g(hipStream_t s, const pool_view& p, const meta_view& m, uint3
     return hipGetLastError();
 }
 
-// Query heads a workgroup covers of a GQA group, and its rows of a tile.
+// Query heads a workgroup covers of a GQA group.
 uint32_t wide_heads(uint32_t group)
 {
     return std::min(group, 4u);

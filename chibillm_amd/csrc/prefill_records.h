@@ -1,22 +1,21 @@
-// The records by which the workgroups that share a prefill tile's keys hand
-// over their partial states (kernels_prefill.hip, kernels_prefill_f32.hip):
-// 16-byte buffer stores and loads with the sc1 cache policy. HIP device code
-// only.
+// The records by which the workgroups that share a prefill tile's keys
+// (kernels_prefill.hip, kernels_prefill_wide.hip, kernels_prefill_f32.hip) or a
+// cut decode row (kernels_decode.hip) hand over their partial states: 16-byte
+// buffer stores and loads with the sc1 cache policy. HIP device code only.
 #pragma once
 
 #include "ckv_internal.h"
 
 namespace ckv {
 
-// The split tiles' records pass between workgroups as the decode's split-K
-// partial records do (kernels_decode.hip), at 16 bytes per access: buffer
-// stores and loads with the sc1 cache policy, the same instructions at the
-// same policy that LLVM emits for relaxed agent-scope atomic stores and loads
-// on gfx950 (global/buffer_store/load sc1: the store writes through, the
-// load misses any L2 line that could be stale, so every XCD sees the data in
-// memory without an L2 writeback); a wait for the stores' completion before
-// one thread's relaxed agent-scope fetch-add counts the share in; the loads
-// of the share that arrives last are issued after that fetch-add returns.
+// Records pass between workgroups at 16 bytes per access: buffer stores and
+// loads with the sc1 cache policy, the same instructions at the same policy
+// that LLVM emits for relaxed agent-scope atomic stores and loads on gfx950
+// (global/buffer_store/load sc1: the store writes through, the load misses any
+// L2 line that could be stale, so every XCD sees the data in memory without an
+// L2 writeback); a wait for the stores' completion before one thread's relaxed
+// agent-scope fetch-add counts the share in; the loads of the share that
+// arrives last are issued after that fetch-add returns.
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "the prefill's split-key handoff relies on gfx950's memory system; build for gfx950"
 #endif
