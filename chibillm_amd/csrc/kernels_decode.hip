@@ -614,7 +614,7 @@ __global__ __launch_bounds__(wide_lanes(G, DT) ? 512 : 1024, wide_lanes(G, DT) ?
             for (int j = 0; j < 4; ++j) {
                 // A lane past the row's end re-read the last token: at weight 0 an
                 // infinite value of it would become NaN, so it takes 0. (Selects
-                // in every unit, at most 1 % of a launch: selects in a branch for
+                // in every unit, at most 1.5 % of a launch: selects in a branch for
                 // the last unit cost 256-wide rows 2.3 % in register copies, a
                 // source of zeros 5.5 % and one long row 6 % in addresses, a copy
                 // of the unit's code spills. f32 words are selected once widened; before,

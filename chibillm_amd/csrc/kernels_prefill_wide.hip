@@ -681,7 +681,8 @@ __global__ __launch_bounds__(64 * waves, 1) void prefill_wide_kernel(
                     make_uint2(pack2<F16>(x[0], x[1]), pack2<F16>(x[2], x[3]));
             }
     }
-    if (__builtin_expect(alone == 0, 1)) // (62.4 us; with the loop in its place 63.3)
+    // (the loop out of the way: 62.4 us in all with two-term probabilities, 63.3 in line)
+    if (__builtin_expect(alone == 0, 1))
         return;
     const size_t first = (size_t)(row0 + rb * 32) * q_stride + (size_t)head * dim;
     for (uint32_t left = alone; left;) {
