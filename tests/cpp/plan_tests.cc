@@ -297,6 +297,24 @@ TEST("small batches: chunks that fit one round of workgroups")
     }
 }
 
+TEST("small f32 batches: two workgroups per compute unit weigh 1.6")
+{
+    auto plan = [](uint32_t rows, uint32_t low, uint32_t high) {
+        std::vector<uint32_t> p(rows);
+        for (uint32_t i = 0; i < rows; ++i)
+            p[i] = low + (uint32_t)((uint64_t)(high - low) * i / (rows - 1)) - 1;
+        return plan_and_check(p, 8, 256, ckv::decode_form_of(CKV_F32, 128)).shape;
+    };
+    // 8 pages for two (12.8) against 14 and 13 for one workgroup per compute unit
+    CHECK(plan(25, 131, 241).split_pages == 8 && plan(27, 64, 242).split_pages == 8);
+    // 8 against 11: one
+    const auto one = plan(8, 300, 900);
+    CHECK(one.split_pages == 11 && one.n_wgs <= 32);
+    // chunks, not dealt out, where dealing takes 0.93 of their time
+    CHECK(!plan(16, 200, 2000).balanced && !plan(20, 1000, 1300).balanced);
+    CHECK(plan(24, 100, 2500).balanced); // 0.87
+}
+
 TEST("more than two units per compute unit: whole rows only where they even out")
 {
     auto whole = [](uint32_t rows, uint32_t low, uint32_t high) {
